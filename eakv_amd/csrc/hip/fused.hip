@@ -548,7 +548,14 @@ __device__ __forceinline__ void merge_unit(const float *pu, int nb, int n_chunks
     else merge_unit_p<D, VS, 2>(pu, nb, n_chunks, G, stage, ou, tid);
 }
 
-// Tile assignment: nb = gridDim.x blocks share one (sequence, kv head), a
+// The chunks of a launch: sequence s has pre[s + 1] - pre[s] of them per
+// virtual kv head, and pre[s] counts those of the sequences before it (entries
+// past the last sequence: the total).
+struct ChunkMap {
+    int32_t pre[EAKVD_MAX_BATCH + 1];
+};
+
+// Tile assignment: nb blocks share one (sequence, kv head), a
 // "unit" of n_tiles TT-token tiles, dealt round robin: tile j to block
 // (j / kWaves) % nb and wave j % kWaves.  At any time the waves of a unit
 // read one contiguous window of every plane, and a wave's tiles are
@@ -568,11 +575,15 @@ __device__ __forceinline__ void merge_unit(const float *pu, int nb, int n_chunks
 // digit rows (signed fixed point, the exponent from the largest |a|); m
 // stays 0, vsum_merge_kernel adds the chunks unnormalised, and a non-finite
 // weight makes its head's output NaN (lsum carries the flag).
+// ch: this block's chunk of the nb of its unit (sequence s, virtual kv head
+// kvh of vkv); blk: its place in the order of dispatch; pre: the chunks per
+// virtual kv head of the sequences before s.
 template <int D, int HH, bool VS, int TT>
-__global__ __launch_bounds__(64 * kWavesH<HH>, (kWavesH<HH> * kBlocksPerCUH<D, HH> / 4)) void mfma_kernel(
-    eakvd_geom g, eakvd_batch bt, int layer, const float *__restrict__ q,
+__device__ __forceinline__ void mfma_body(
+    const eakvd_geom &g, const eakvd_batch &bt, int layer, const float *__restrict__ q,
     int n_q, int qpk, float rs, float *__restrict__ part, int split,
-    float *__restrict__ out, uint8_t *__restrict__ ctr, int lead)
+    float *__restrict__ out, uint8_t *__restrict__ ctr, int lead_from,
+    int ch, int nb, int kvh, int vkv, int s, int pre, int blk)
 {
     constexpr int GPD = D / 64;
     constexpr int NK = Geo<D, TT>::NK;
@@ -596,8 +607,14 @@ __global__ __launch_bounds__(64 * kWavesH<HH>, (kWavesH<HH> * kBlocksPerCUH<D, H
     __shared__ __attribute__((aligned(16))) float s_lds1[NW][Geo<D, TT>::SSLOT];
     __shared__ __attribute__((aligned(16))) uint8_t z_lds[NW][HH * Geo<D, TT>::ZROWS * 8];
 
-    const int ch = blockIdx.x, nb = gridDim.x, kvh = blockIdx.y, s = blockIdx.z;
     const int L = bt.seq_len[s];
+    const uint8_t *base = bt.base[s];
+    // Every kernel argument that the first loads need, read at once: the
+    // compiler otherwise reads them where they are used, one scalar load round
+    // trip after another before the first K and V bytes are requested.
+    asm volatile("" ::"s"(L), "s"(base), "s"(layer), "s"(q), "s"(n_q), "s"(qpk), "s"(split), "s"(nb),
+                 "s"(vkv), "s"(pre), "s"(g.gph), "s"(g.max_groups), "s"(g.s_off), "s"(g.b_off),
+                 "s"(g.block_bytes), "s"(ctr), "s"(lead_from), "s"(part), "s"(rs), "s"(out));
     const int n_tiles = (L + TT - 1) / TT;
     if (ch * NW >= n_tiles) {         // no tile for this block: no partial
         // merged here, an empty sequence's outputs are 0 * (1/0) = NaN, as
@@ -617,8 +634,8 @@ __global__ __launch_bounds__(64 * kWavesH<HH>, (kWavesH<HH> * kBlocksPerCUH<D, H
     const int G = qpk;                                  // 1..4 HH
     const int first = ch * NW + w;                      // this wave's first tile
     const int stride = nb * NW;                         // tiles between its tiles
-    const Planes K = planes_of(g, bt.base[s], layer, 0);
-    const Planes V = planes_of(g, bt.base[s], layer, 1);
+    const Planes K = planes_of(g, base, layer, 0);
+    const Planes V = planes_of(g, base, layer, 1);
     // split > 1: blockIdx.y is one of `split` virtual kv heads of qpk q heads
     // each that share kv head kvh / split (more than 8 q heads per kv head)
     const int64_t hbase = (int64_t)(kvh / split) * g.gph;
@@ -1129,18 +1146,17 @@ __global__ __launch_bounds__(64 * kWavesH<HH>, (kWavesH<HH> * kBlocksPerCUH<D, H
     constexpr int kGrp = Geo<D, TT>::NVD + kDma<D, TT> + NKL;   // loads per group
     constexpr int kLater = (kSlots - 1) * kGrp;         // loads of the groups after the oldest
     constexpr int kEarly = (kSlots - 2) * kGrp;
-    // lead > 0 (one-quad waves): the grid holds two blocks per CU, dealt one
-    // per CU in each of two dispatch rounds (blocks in linear order), and on
-    // each SIMD the older wave wins issue, so the first round's blocks would
+    // lead_from > 0 (one-quad waves): the grid holds two blocks per CU, dealt
+    // one per CU in each of two dispatch rounds (blocks in linear order), and
+    // on each SIMD the older wave wins issue, so the first round's blocks would
     // run ahead and the second's finish alone at half the CU's rate.  The
-    // second round's waves issue first for their first `lead` tiles (half of
-    // them), then give way.  Priority changes no arithmetic.
+    // second round's waves (blocks lead_from and later) issue first for the
+    // first half of their tiles, then give way.  Priority changes no
+    // arithmetic.
     if constexpr (HH == 1)
-        if (lead > 0 &&
-            2 * (int)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) >=
-                (int)(gridDim.x * gridDim.y * gridDim.z)) {
-            lead_left = lead;
-            __builtin_amdgcn_s_setprio(1);
+        if (lead_from > 0 && blk >= lead_from) {
+            lead_left = ((n_tiles - first + stride - 1) / stride + 1) / 2;
+            if (lead_left > 0) __builtin_amdgcn_s_setprio(1);
         }
     if (tk[0] < n_tiles) {
         {
@@ -1253,7 +1269,7 @@ __global__ __launch_bounds__(64 * kWavesH<HH>, (kWavesH<HH> * kBlocksPerCUH<D, H
             o0 = fmaf(ov.x, f, o0);
             o1 = fmaf(ov.y, f, o1);
         }
-        float *dst = part + (((int64_t)s * n_q + kvh * qpk + h) * nb + ch) * (D + 2);
+        float *dst = part + ((int64_t)pre * n_q + (kvh * qpk + h) * nb + ch) * (D + 2);
         if (ctr) {
             st_dev2(dst + 2 + dim, o0, o1);
             if (dim == 0) st_dev2(dst, M, lt);
@@ -1274,7 +1290,7 @@ __global__ __launch_bounds__(64 * kWavesH<HH>, (kWavesH<HH> * kBlocksPerCUH<D, H
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     unsigned *uc = reinterpret_cast<unsigned *>(
-        ctr + ((int64_t)s * gridDim.y + kvh) * EAKVD_CTR_STRIDE);
+        ctr + ((int64_t)s * vkv + kvh) * EAKVD_CTR_STRIDE);
     if (tid == 0)
         ((int *)z_lds[0])[0] = __hip_atomic_fetch_add(uc, 1u, __ATOMIC_RELAXED,
                                                       __HIP_MEMORY_SCOPE_AGENT) ==
@@ -1284,9 +1300,41 @@ __global__ __launch_bounds__(64 * kWavesH<HH>, (kWavesH<HH> * kBlocksPerCUH<D, H
     if (tid == 0) __hip_atomic_store(uc, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     static_assert(4 * HH * D / 2 <= 64 * NW && 4 * HH * kInBatch <= 64 * NW,
                   "one output pair and at most one (m, l) pair per thread");
-    const int64_t qh0 = (int64_t)s * n_q + kvh * qpk;
-    merge_unit<D, VS>(part + qh0 * nb * (D + 2), nb, n_chunks, G, &s_lds0[0][0],
-                      out + qh0 * D, tid, 64 * NW);
+    merge_unit<D, VS>(part + ((int64_t)pre * n_q + kvh * qpk * nb) * (D + 2), nb, n_chunks, G,
+                      &s_lds0[0][0], out + ((int64_t)s * n_q + kvh * qpk) * D, tid, 64 * NW);
+}
+
+// Every sequence in gridDim.x chunks: the grid is (chunk, virtual kv head,
+// sequence).
+template <int D, int HH, bool VS, int TT>
+__global__ __launch_bounds__(64 * kWavesH<HH>, (kWavesH<HH> * kBlocksPerCUH<D, HH> / 4)) void mfma_kernel(
+    eakvd_geom g, eakvd_batch bt, int layer, const float *__restrict__ q,
+    int n_q, int qpk, float rs, float *__restrict__ part, int split,
+    float *__restrict__ out, uint8_t *__restrict__ ctr, int lead_from)
+{
+    const int ch = blockIdx.x, nb = gridDim.x, kvh = blockIdx.y, vkv = gridDim.y, s = blockIdx.z;
+    mfma_body<D, HH, VS, TT>(g, bt, layer, q, n_q, qpk, rs, part, split, out, ctr, lead_from, ch,
+                             nb, kvh, vkv, s, s * nb, (s * vkv + kvh) * nb + ch);
+}
+
+// Contexts of several lengths: a one-dimensional grid, dealt by cm.  A kernel
+// of its own: with one kernel for both, the launches of one sequence waited
+// for the map's first load before their others (8Q/8KV d128 at 2048 tokens
+// and 32Q/4KV d64 at 4096: 0.4-0.5 us more per call).
+template <int D, int HH, int TT>
+__global__ __launch_bounds__(64 * kWavesH<HH>, (kWavesH<HH> * kBlocksPerCUH<D, HH> / 4)) void ragged_kernel(
+    eakvd_geom g, eakvd_batch bt, ChunkMap cm, int layer, const float *__restrict__ q,
+    int n_q, int qpk, float rs, float *__restrict__ part, int split,
+    float *__restrict__ out, uint8_t *__restrict__ ctr, int vkv, int lead_from)
+{
+    const int blk = blockIdx.x;
+    int s = 0;
+#pragma unroll
+    for (int i = 1; i < EAKVD_MAX_BATCH; i++) s += blk >= cm.pre[i] * vkv;
+    const int pre = cm.pre[s], nb = cm.pre[s + 1] - pre;
+    const int r = blk - pre * vkv, kvh = r / nb;
+    mfma_body<D, HH, false, TT>(g, bt, layer, q, n_q, qpk, rs, part, split, out, ctr, lead_from,
+                                r - kvh * nb, nb, kvh, vkv, s, pre, blk);
 }
 
 // Merge of the MFMA program's chunk partials (log2 domain) per (q head,
@@ -1299,15 +1347,16 @@ constexpr int kMergeBatch = 16;
 
 template <int D>
 __global__ __launch_bounds__(D) void merge_kernel(
-    eakvd_batch bt, int n_q, int max_chunks, int wpb, int tt, const float *__restrict__ part,
+    eakvd_batch bt, ChunkMap cm, int n_q, int wpb, int tt, const float *__restrict__ part,
     float *__restrict__ out)
 {
     const int qh = blockIdx.x, s = blockIdx.y, i = threadIdx.x;
     // blocks that had a tile (see mfma_kernel; wpb waves per block, tt
     // tokens per tile)
+    const int max_chunks = cm.pre[s + 1] - cm.pre[s];
     const int n_tiles = (bt.seq_len[s] + tt - 1) / tt;
     const int n_chunks = min(max_chunks, (n_tiles + wpb - 1) / wpb);
-    const float *p = part + ((int64_t)s * n_q + qh) * max_chunks * (D + 2);
+    const float *p = part + ((int64_t)cm.pre[s] * n_q + qh * max_chunks) * (D + 2);
     // The (m, l) pair and o[i] of every chunk by vector buffer loads, all
     // issued before any arithmetic: one memory round trip.  (As scalar
     // loads the pairs overflow the scalar load counter, and the compiler's
@@ -1353,7 +1402,7 @@ constexpr int kPartBatch = 8;
 
 template <int D>
 __global__ __launch_bounds__(256) void merge_parts_kernel(
-    eakvd_batch bt, int n_q, int max_chunks, int wpb, int tt, const float *__restrict__ part,
+    eakvd_batch bt, ChunkMap cm, int n_q, int wpb, int tt, const float *__restrict__ part,
     float *__restrict__ out)
 {
     __shared__ float pm[kMergeParts], pl[kMergeParts], po[kMergeParts][32];
@@ -1361,9 +1410,10 @@ __global__ __launch_bounds__(256) void merge_parts_kernel(
     const int i = (blockIdx.x % (D / 32)) * 32 + (threadIdx.x & 31), pt = threadIdx.x >> 5;
     // blocks that had a tile (see mfma_kernel; wpb waves per block, tt
     // tokens per tile)
+    const int max_chunks = cm.pre[s + 1] - cm.pre[s];
     const int n_tiles = (bt.seq_len[s] + tt - 1) / tt;
     const int n_chunks = min(max_chunks, (n_tiles + wpb - 1) / wpb);
-    const float *p = part + ((int64_t)s * n_q + qh) * max_chunks * (D + 2);
+    const float *p = part + ((int64_t)cm.pre[s] * n_q + qh * max_chunks) * (D + 2);
     float M = -1000000.0f * EAKV_LOG2E, lt = 0.0f, ot = 0.0f;
     for (int c0 = pt; c0 < n_chunks; c0 += kMergeParts * kPartBatch) {
         float m[kPartBatch], lv[kPartBatch], ov[kPartBatch];
@@ -1728,6 +1778,16 @@ auto mfma_entry(int d, int hh, int tt)
     return tt == 64 ? mfma_kernel<128, 2, VS, 64> : mfma_kernel<128, 2, VS, 32>;
 }
 
+auto ragged_entry(int d, int hh, int tt)
+{
+    if (d == 64) {
+        if (hh == 1) return ragged_kernel<64, 1, 32>;
+        return tt == 64 ? ragged_kernel<64, 2, 64> : ragged_kernel<64, 2, 32>;
+    }
+    if (hh == 1) return ragged_kernel<128, 1, 32>;
+    return tt == 64 ? ragged_kernel<128, 2, 64> : ragged_kernel<128, 2, 32>;
+}
+
 // The launch shape of one fused call: the matrix-core program (chunks per
 // unit mc, waves per block wpb, virtual kv heads per kv head split, q heads
 // per virtual head qv, quads hh, tokens per tile tt) or the VALU program
@@ -1735,7 +1795,77 @@ auto mfma_entry(int d, int hh, int tt)
 struct FusedPlan {
     bool mfma;
     int mc, wpb, split, qv, hh, tt;
+    bool even;          // every sequence of the batch in mc chunks
+    ChunkMap cm;        // else mc is the most of a sequence
 };
+
+// cm with mc chunks for each of n sequences
+void even_chunks(ChunkMap *cm, int n, int mc)
+{
+    for (int i = 0; i <= EAKVD_MAX_BATCH; i++) cm->pre[i] = (i < n ? i : n) * mc;
+}
+
+// Chunks for contexts of several lengths.  With as many chunks for every
+// sequence the longest context decides the call while the blocks of the short
+// ones idle; here a chunk covers about the same tokens in every sequence, R
+// rounds of the block's waves (wpb * tt tokens a round), R the smallest for
+// which the chunks fit the resident blocks (`slots`).
+//  - A chunk holds at least 4 * kChunkM tokens, as in mfma_blocks_per_unit.
+//  - Up to kInBatch chunks of a unit are merged in the launch; two rounds more
+//    are cheaper than the merge launch (about 3 us), so R goes up to that.
+//  - Whole chunks leave slots idle where there are few per sequence.  From 8
+//    rounds on, where a quarter more than the even share would be taken, the
+//    chunks may exceed the slots: by half for one quad (its registers and LDS
+//    let three blocks share a CU), to twice for two quads (a second round of
+//    dispatch).
+// Measured (us per layer; chunks of the longest context for all, against
+// these): 32Q/8KV d128, 24 contexts of 283-12289 tokens, 46.2 against 33.7; 12
+// of 1031-60000, 88 against 53; 64Q/8KV d128, 30 of 291-13656, 69 against 44, 6
+// of 5003-20000, 29.2 against 22.6; 40Q/8KV, 14 up to 20000, 52 against 24.
+// Contexts that differ little keep the even deal, whose more and smaller
+// blocks end as early (32Q/8KV, 9 of 1097-3000: 11.6 against 12.6 us; 32Q/4KV
+// d64, 32 of 1250-5000: 17.1 against 17.7): two rounds of 128-dim tokens must
+// be saved, and a quarter.
+// Returns the most chunks of a sequence, or 0 to keep the even deal, whose
+// blocks take even_rounds.
+int ragged_chunks(ChunkMap *cm, const eakvd_batch *b, int vkv, int slots, int round, int hh,
+                  int gpd, int even_rounds)
+{
+    const int n = b->n_seq;
+    int64_t sum = 0;
+    int most = 1;                                          // rounds of the longest context
+    int rounds[EAKVD_MAX_BATCH];
+    for (int i = 0; i < n; i++) {
+        rounds[i] = b->seq_len[i] > 0 ? (b->seq_len[i] + round - 1) / round : 1;
+        most = rounds[i] > most ? rounds[i] : most;
+        sum += rounds[i];
+    }
+    auto fit = [&](int64_t budget) {
+        // from an even share of all rounds (or the least chunk) to the
+        // longest context in one chunk
+        int lo = (int)(sum / (budget < 1 ? 1 : budget)), hi = most;
+        const int least = (4 * kChunkM + round - 1) / round;
+        lo = lo < least ? least : lo;
+        hi = hi < lo ? lo : hi;
+        while (lo < hi) {
+            const int mid = lo + (hi - lo) / 2;
+            int64_t t = 0;
+            for (int i = 0; i < n; i++) t += (rounds[i] + mid - 1) / mid;
+            if (t <= budget) hi = mid;
+            else lo = mid + 1;
+        }
+        const int one_launch = (most + kInBatch - 1) / kInBatch;
+        return lo < one_launch && one_launch <= lo + 2 ? one_launch : lo;
+    };
+    int r = fit(slots / vkv);
+    if (r >= 8 && 4 * (int64_t)r * slots >= 5 * sum * vkv)
+        r = fit((hh == 1 ? slots + slots / 2 : 2 * slots) / vkv);
+    if (4 * r > 3 * even_rounds || (even_rounds - r) * gpd < 4) return 0;
+    cm->pre[0] = 0;
+    for (int i = 0; i < EAKVD_MAX_BATCH; i++)
+        cm->pre[i + 1] = cm->pre[i] + (i < n ? (rounds[i] + r - 1) / r : 0);
+    return (most + r - 1) / r;
+}
 
 FusedPlan fused_plan(const eakvd_geom *g, const eakvd_batch *b, int n_q, int n_kv)
 {
@@ -1754,6 +1884,17 @@ FusedPlan fused_plan(const eakvd_geom *g, const eakvd_batch *b, int n_q, int n_k
         p.wpb = p.hh == 1 ? kWavesH<1> : kWavesH<2>;
         p.mc = mfma_blocks_per_unit(ml, b->n_seq * n_kv * p.split, per_cu);
         p.tt = tile_tokens(p.hh, ml, p.mc, p.wpb);
+        bool ragged = false;
+        for (int i = 1; i < b->n_seq; i++) ragged = ragged || b->seq_len[i] != b->seq_len[0];
+        int mc = 0;
+        if (ragged) {
+            const int round = p.wpb * p.tt;
+            mc = ragged_chunks(&p.cm, b, n_kv * p.split, cu_count() * per_cu, round, p.hh,
+                               (int)g->gpd, (ml + round * p.mc - 1) / (round * p.mc));
+        }
+        p.even = mc == 0;
+        if (p.even) even_chunks(&p.cm, b->n_seq, p.mc);
+        else p.mc = mc;
     } else {
         p.mc = (ml + kChunkV - 1) / kChunkV;
     }
@@ -1775,7 +1916,8 @@ extern "C" size_t eakvd_fused_launch_bytes(const eakvd_geom *g, const eakvd_batc
 {
     // partial (m, l, o[D]) of every (sequence, q head, chunk)
     const FusedPlan p = fused_plan(g, b, n_q, n_kv);
-    return (size_t)b->n_seq * n_q * p.mc * (g->head_dim + 2) * sizeof(float);
+    const size_t chunks = p.mfma ? (size_t)p.cm.pre[b->n_seq] : (size_t)b->n_seq * p.mc;
+    return chunks * n_q * (g->head_dim + 2) * sizeof(float);
 }
 
 extern "C" int eakvd_scratch(void **p)
@@ -1813,17 +1955,20 @@ extern "C" void eakvd_fused_plan(const eakvd_geom *g, const eakvd_batch *b, int 
                                  const void *ctr, int32_t *out)
 {
     const FusedPlan p = fused_plan(g, b, n_q, n_kv);
-    const int ml = max_len(b);
     out[0] = p.mfma;
     out[1] = p.mc;
     if (p.mfma) {
         const int64_t units = (int64_t)n_kv * p.split * b->n_seq;
-        const int64_t n_tiles = ((int64_t)ml + p.tt - 1) / p.tt;
-        const int64_t waves = (int64_t)p.mc * p.wpb;
         out[2] = merge_in_launch(g, ctr, p.mc, units);
         out[3] = p.tt;
         out[4] = p.wpb;
-        out[5] = (int32_t)((n_tiles + waves - 1) / waves);
+        out[5] = 0;
+        for (int i = 0; i < b->n_seq; i++) {
+            const int64_t n_tiles = ((int64_t)b->seq_len[i] + p.tt - 1) / p.tt;
+            const int64_t waves = (int64_t)(p.cm.pre[i + 1] - p.cm.pre[i]) * p.wpb;
+            const int32_t t = (int32_t)((n_tiles + waves - 1) / waves);
+            out[5] = t > out[5] ? t : out[5];
+        }
         out[6] = p.hh;
         out[7] = p.split;
     } else {
@@ -1846,12 +1991,12 @@ extern "C" int eakvd_fused(const eakvd_geom *g, const eakvd_batch *b,
     const FusedPlan p = fused_plan(g, b, n_q, n_kv);
     if (p.mfma) {
         const int mc = p.mc, wpb = p.wpb, hh = p.hh;
-        const dim3 grid((unsigned)mc, (unsigned)(n_kv * p.split), (unsigned)b->n_seq);
+        const int vkv = n_kv * p.split;
+        const int blocks = p.cm.pre[b->n_seq] * vkv;
         const dim3 mgrid((unsigned)n_q, (unsigned)b->n_seq);
         // more than one batch of chunks: the merge spread over 8 parts
         const bool parts = mc > kMergeBatch;
         const dim3 pgrid((unsigned)(n_q * (g->head_dim / 32)), (unsigned)b->n_seq);
-        auto kern = mfma_entry<false>(g->head_dim, hh, p.tt);
         const int64_t units = (int64_t)n_kv * p.split * b->n_seq;
         uint8_t *uc = merge_in_launch(g, ctr, mc, units) ? (uint8_t *)ctr : nullptr;
         // one-quad grids of exactly two rounds of one block per CU: the
@@ -1859,27 +2004,29 @@ extern "C" int eakvd_fused(const eakvd_geom *g, const eakvd_batch *b,
         // 54.48-54.51 against 55.07-55.13 us per layer step, alternating
         // whole bench runs on one box; 55.24-55.30 against 55.55-55.96 on
         // another)
-        int lead = 0;
-        if (hh == 1 && units * mc == 2 * (int64_t)cu_count()) {
-            const int64_t n_tiles = ((int64_t)max_len(b) + p.tt - 1) / p.tt;
-            const int64_t waves = (int64_t)mc * wpb;
-            lead = (int)(((n_tiles + waves - 1) / waves + 1) / 2);
-        }
-        hipLaunchKernelGGL(kern, grid, dim3(64 * wpb), 0, st, *g, *b, layer, q, n_q, p.qv, rs,
-                           part, p.split, out, uc, lead);
+        const int lead_from = hh == 1 && blocks == 2 * cu_count() ? cu_count() : 0;
+        if (p.even)
+            hipLaunchKernelGGL(mfma_entry<false>(g->head_dim, hh, p.tt),
+                               dim3((unsigned)mc, (unsigned)vkv, (unsigned)b->n_seq),
+                               dim3(64 * wpb), 0, st, *g, *b, layer, q, n_q, p.qv, rs, part,
+                               p.split, out, uc, lead_from);
+        else
+            hipLaunchKernelGGL(ragged_entry(g->head_dim, hh, p.tt), dim3((unsigned)blocks),
+                               dim3(64 * wpb), 0, st, *g, *b, p.cm, layer, q, n_q, p.qv, rs,
+                               part, p.split, out, uc, vkv, lead_from);
         if (uc) return (int)hipGetLastError();
         const int tt = p.tt;
         if (parts && g->head_dim == 64)
-            hipLaunchKernelGGL(merge_parts_kernel<64>, pgrid, dim3(256), 0, st, *b, n_q, mc,
+            hipLaunchKernelGGL(merge_parts_kernel<64>, pgrid, dim3(256), 0, st, *b, p.cm, n_q,
                                wpb, tt, part, out);
         else if (parts)
-            hipLaunchKernelGGL(merge_parts_kernel<128>, pgrid, dim3(256), 0, st, *b, n_q, mc,
+            hipLaunchKernelGGL(merge_parts_kernel<128>, pgrid, dim3(256), 0, st, *b, p.cm, n_q,
                                wpb, tt, part, out);
         else if (g->head_dim == 64)
-            hipLaunchKernelGGL(merge_kernel<64>, mgrid, dim3(64), 0, st, *b, n_q, mc, wpb,
+            hipLaunchKernelGGL(merge_kernel<64>, mgrid, dim3(64), 0, st, *b, p.cm, n_q, wpb,
                                tt, part, out);
         else
-            hipLaunchKernelGGL(merge_kernel<128>, mgrid, dim3(128), 0, st, *b, n_q, mc, wpb,
+            hipLaunchKernelGGL(merge_kernel<128>, mgrid, dim3(128), 0, st, *b, p.cm, n_q, wpb,
                                tt, part, out);
         return (int)hipGetLastError();
     }

@@ -1,0 +1,55 @@
+"""Batches of several context lengths on the fused call's proportional chunks.
+
+A batch whose contexts differ enough gives each sequence chunks in proportion
+to its length (ragged_kernel, hip/fused.hip) instead of as many chunks for all.
+Each case names its chunks of the longest context on 256 CUs and covers an edge:
+contexts of one token, around a tile (32) and a round of a block (128), an
+empty sequence, more than 16 chunks of a unit (the merge launch), more blocks
+than the chip holds at once, two quads, both head_dims, groups split into
+virtual kv heads.  Outputs are held to the reference bar
+(fused_attention.ea:190-373), both entry points to the same bits.
+"""
+import numpy as np
+import pytest
+
+from test_gpu_headline import (E, batch_call, build_batch, chan_k,  # noqa: F401
+                               compare_sequences, n_cu, say)
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    (128, 8, 32, [9001, 1, 31, 32, 33, 127, 128, 129, 4000], 15),
+    (64, 8, 32, [50000, 1, 500], 56),
+    (128, 8, 8, [7000] + [200] * 20, 14),
+    (128, 8, 64, [12000] + [300 + i for i in range(29)], 12),
+    (128, 8, 40, [30000, 100], 15),
+    (64, 4, 32, [30000, 257, 1, 3000, 33], None),
+    (128, 2, 64, [10000, 64, 65], 14),
+]
+
+
+@pytest.mark.parametrize("d,n_kv,n_q,lens,chunks", CASES)
+def test_ragged_batch(E, d, n_kv, n_q, lens, chunks):  # noqa: F811
+    say("ragged: build", d, n_q, n_kv, lens)
+    gs, os_ = build_batch(E, 0xEA4B + 700 + d + len(lens), len(lens), n_kv, d, lens,
+                          max(lens) + 3, chan_k)
+    empty = E.Cache(1, n_kv, d, max(lens) + 3)
+    n = len(gs) + 1
+    batch = gs[:1] + [empty] + gs[1:]
+    plan = E.fused_plan(batch, n_q, n_kv)
+    say("ragged: plan", plan)
+    if n_cu() == 256:
+        assert plan["mfma"] == 1 and chunks in (None, plan["chunks"])
+        assert plan["merge_levels"] == (1 if plan["chunks"] <= 16 else 0)
+    rng = np.random.default_rng(0xEA4B + 701 + d)
+    q = rng.standard_normal((n, n_q, d), dtype=np.float32)
+    out = batch_call(E, "eakv_attention_fused_batch_device", batch, q, n_q, n_kv)
+    out_na = batch_call(E, "eakv_attention_fused_batch_device_noalloc", batch, q, n_q, n_kv)
+    again = batch_call(E, "eakv_attention_fused_batch_device", batch, q, n_q, n_kv)
+    keep = [0] + list(range(2, n))
+    assert np.array_equal(out[keep].view(np.uint32), out_na[keep].view(np.uint32))
+    assert np.array_equal(out[keep].view(np.uint32), again[keep].view(np.uint32))
+    assert all(np.isnan(x[1]).all() for x in (out, out_na, again))
+    compare_sequences(os_, q[keep], out[keep], n_q, n_kv, lens)
+    for g in batch:
+        g.free()
