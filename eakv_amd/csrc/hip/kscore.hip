@@ -11,8 +11,9 @@
 //
 // Layout: one lane per token.  A token's 32*gpd packed bytes are read as
 // uint4 vectors; its dequantized values are computed once and dotted with
-// every q head of its group (the reference GQA loop flip).  The q vectors are
-// wave-uniform and are read through the scalar cache.  Each block walks
+// every q head of its group (the reference GQA loop flip): groups of q heads on
+// the matrix cores (k_score_mfma_kernel), one q head per kv head by vector
+// FMAs.  Each block walks
 // several 256-token slices with the next slice's loads in flight while it
 // computes the current one.  Nibbles become floats by masking a dword to four
 // byte-wide nibbles and converting its bytes (v_cvt_f32_ubyte0..3): exact,
@@ -26,14 +27,6 @@ namespace {
 
 constexpr int kKsBufs = 2;                          // slices per wave in flight, one consumed
 constexpr int kKsBlocksPerCU = 2;
-
-template <int J>
-__device__ __forceinline__ void dequant4(float *klo, float *khi, uint32_t lo, uint32_t hi,
-                                         float s, float b)
-{
-    klo[J] = fmaf(ubyte_f32<J>(lo), s, b);
-    khi[J] = fmaf(ubyte_f32<J>(hi), s, b);
-}
 
 template <int D>
 struct KTok {
@@ -79,97 +72,58 @@ __device__ __forceinline__ void k_load(const uint8_t *w, const float *sc, const 
     }
 }
 
-// Block b takes the 256-token slices b, b + gridDim.x, ... of its kv head
-// (one token per lane) and loads the next slice while it computes one.
-template <int D, bool MHA>
-__device__ __forceinline__ void k_score_body(
+// One q head per kv head, one lane per token: registers for 2 waves per
+// SIMD.  Long contexts: its 16-byte loads read a token's row at once.  Block b
+// takes the 256-token slices b, b + gridDim.x, ... of its kv head and loads
+// the next slice while it computes one.
+template <int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void k_score_mha_kernel(
     const uint8_t *__restrict__ kw, const float *__restrict__ ks,
     const float *__restrict__ kb, int64_t gph, int L,
-    const float *__restrict__ q, int qpk, float *__restrict__ scores, float rs)
+    const float *__restrict__ q, float *__restrict__ scores, float rs)
 {
     constexpr int GPD = D / 64;
-    constexpr int NC = D / 16;
     const int kvh = blockIdx.y;
     const int n_sl = (L + 255) / 256;
     const int64_t hb = (int64_t)kvh * gph;        // the kv head's first group
     const uint8_t *hw = kw + hb * 32;
     const float *hs = ks + hb, *hbi = kb + hb;
-    const float *qk = q + (int64_t)kvh * qpk * D;
-    // blockIdx.z: which of gridDim.z equal parts of the group's q heads
-    // this block dots (a grid too small for the chip splits the heads)
-    const int qn = qpk / (int)gridDim.z, o0 = (int)blockIdx.z * qn;
+    const float *qk = q + (int64_t)kvh * D;
 
-    // one 256-token slice: dequantize each lane's token once, then dot it
-    // with every q head of the kv head in this block's part
     auto compute = [&](const KTok<D> &T, int sl) {
         const int t = sl * 256 + threadIdx.x;
-        if constexpr (MHA) {
-            // one q head: each dequantized value goes straight into its fma,
-            // chunks c = 4*grp + 2*nib + half in order
-            float acc[16];
+        // each dequantized value goes straight into its fma, chunks
+        // c = 4*grp + 2*nib + half in order
+        float acc[16];
 #pragma unroll
-            for (int i = 0; i < 16; i++) acc[i] = 0.0f;
-            // q is read through the scalar cache per slice: the compiler
-            // barrier keeps it from holding all D values in vector registers
-            // across slices
-            const float *qh = qk;
-            asm volatile("" ::: "memory");
-#pragma unroll
-            for (int grp = 0; grp < GPD; grp++)
-#pragma unroll
-                for (int nib = 0; nib < 2; nib++)
-#pragma unroll
-                    for (int half = 0; half < 2; half++) {
-                        const uint4 v = T.raw[grp * 2 + half];
-                        const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
-                        const float *qc = qh + (4 * grp + 2 * nib + half) * 16;
-#pragma unroll
-                        for (int wd = 0; wd < 4; wd++) {
-                            const uint32_t n = (nib ? w4[wd] >> 4 : w4[wd]) & 0x0f0f0f0fu;
-                            float *a = &acc[4 * wd];
-                            const float s = T.sc[grp], b = T.bi[grp];
-                            a[0] = fmaf(fmaf(ubyte_f32<0>(n), s, b), qc[4 * wd + 0], a[0]);
-                            a[1] = fmaf(fmaf(ubyte_f32<1>(n), s, b), qc[4 * wd + 1], a[1]);
-                            a[2] = fmaf(fmaf(ubyte_f32<2>(n), s, b), qc[4 * wd + 2], a[2]);
-                            a[3] = fmaf(fmaf(ubyte_f32<3>(n), s, b), qc[4 * wd + 3], a[3]);
-                        }
-                    }
-            if (t < L) scores[(int64_t)kvh * L + t] = __fmul_rn(reduce16(acc), rs);
-            return;
-        }
-        // k[c*16 + i]: chunk c = 4*grp + 2*nib + half, byte i of half `half`
-        float k[D];
+        for (int i = 0; i < 16; i++) acc[i] = 0.0f;
+        // q is read through the scalar cache per slice: the compiler
+        // barrier keeps it from holding all D values in vector registers
+        // across slices
+        const float *qh = qk;
+        asm volatile("" ::: "memory");
 #pragma unroll
         for (int grp = 0; grp < GPD; grp++)
 #pragma unroll
-            for (int half = 0; half < 2; half++) {
-                const uint4 v = T.raw[grp * 2 + half];
-                const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+            for (int nib = 0; nib < 2; nib++)
 #pragma unroll
-                for (int wd = 0; wd < 4; wd++) {
-                    const uint32_t lo = w4[wd] & 0x0f0f0f0fu;
-                    const uint32_t hi = (w4[wd] >> 4) & 0x0f0f0f0fu;
-                    float *klo = &k[(4 * grp + half) * 16 + 4 * wd];
-                    float *khi = &k[(4 * grp + 2 + half) * 16 + 4 * wd];
-                    dequant4<0>(klo, khi, lo, hi, T.sc[grp], T.bi[grp]);
-                    dequant4<1>(klo, khi, lo, hi, T.sc[grp], T.bi[grp]);
-                    dequant4<2>(klo, khi, lo, hi, T.sc[grp], T.bi[grp]);
-                    dequant4<3>(klo, khi, lo, hi, T.sc[grp], T.bi[grp]);
+                for (int half = 0; half < 2; half++) {
+                    const uint4 v = T.raw[grp * 2 + half];
+                    const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+                    const float *qc = qh + (4 * grp + 2 * nib + half) * 16;
+#pragma unroll
+                    for (int wd = 0; wd < 4; wd++) {
+                        const uint32_t n = (nib ? w4[wd] >> 4 : w4[wd]) & 0x0f0f0f0fu;
+                        float *a = &acc[4 * wd];
+                        const float s = T.sc[grp], b = T.bi[grp];
+                        a[0] = fmaf(fmaf(ubyte_f32<0>(n), s, b), qc[4 * wd + 0], a[0]);
+                        a[1] = fmaf(fmaf(ubyte_f32<1>(n), s, b), qc[4 * wd + 1], a[1]);
+                        a[2] = fmaf(fmaf(ubyte_f32<2>(n), s, b), qc[4 * wd + 2], a[2]);
+                        a[3] = fmaf(fmaf(ubyte_f32<3>(n), s, b), qc[4 * wd + 3], a[3]);
+                    }
                 }
-            }
-        for (int o = o0; o < o0 + qn; o++) {
-            const float *qv = qk + (int64_t)o * D;
-            float acc[16];
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[i] = 0.0f;
-#pragma unroll
-            for (int c = 0; c < NC; c++)
-#pragma unroll
-                for (int i = 0; i < 16; i++)
-                    acc[i] = fmaf(k[c * 16 + i], qv[c * 16 + i], acc[i]);
-            if (t < L)
-                scores[(int64_t)(kvh * qpk + o) * L + t] = __fmul_rn(reduce16(acc), rs);
-        }
+        if (t < L) scores[(int64_t)kvh * L + t] = __fmul_rn(reduce16(acc), rs);
     };
 
     // kKsBufs buffers in turn: the next kKsBufs - 1 slices load while one is
@@ -191,27 +145,6 @@ __device__ __forceinline__ void k_score_body(
             if (sl >= n_sl) return;
         }
     }
-}
-
-template <int D>
-__global__ __launch_bounds__(256) void k_score_kernel(
-    const uint8_t *__restrict__ kw, const float *__restrict__ ks,
-    const float *__restrict__ kb, int64_t gph, int L,
-    const float *__restrict__ q, int qpk, float *__restrict__ scores, float rs)
-{
-    k_score_body<D, false>(kw, ks, kb, gph, L, q, qpk, scores, rs);
-}
-
-// One q head per kv head, one lane per token: registers for 2 waves per
-// SIMD.  Long contexts: its 16-byte loads read a token's row at once.
-template <int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-void k_score_mha_kernel(
-    const uint8_t *__restrict__ kw, const float *__restrict__ ks,
-    const float *__restrict__ kb, int64_t gph, int L,
-    const float *__restrict__ q, int qpk, float *__restrict__ scores, float rs)
-{
-    k_score_body<D, true>(kw, ks, kb, gph, L, q, qpk, scores, rs);
 }
 
 // One q head per kv head (MHA), short contexts: four lanes per token.  Lane part j of a
@@ -319,7 +252,7 @@ __global__ __launch_bounds__(256) void k_score_mha4_kernel(
         if (j == 0 && t < L) scores[(int64_t)kvh * L + t] = __fmul_rn(v1, rs);
     };
 
-    // as k_score_body: kMhaBufs buffers in turn, the loads past the last
+    // as k_score_mha_kernel: kMhaBufs buffers in turn, the loads past the last
     // slice unconditional (0, no memory traffic)
     const int G = gridDim.x;
     KQuad<D> buf[kMhaBufs];
@@ -338,27 +271,149 @@ __global__ __launch_bounds__(256) void k_score_mha4_kernel(
     }
 }
 
-// Blocks per kv head: two waves per SIMD over the chip, at most one per
-// 256-token slice.
-int k_blocks(int n_sl, int n_kv)
+// Groups of q heads: the dots on the matrix cores, bit for bit the reference's.
+// v_mfma_f32_4x4x1_16b_f32 adds to 16 blocks of 4x4 values one product each, a
+// fused multiply-add with one rounding (denormals kept): with K = 1 a chain of
+// them is the reference's accumulator chain.  Block b of the instruction holds
+// the lanes' tokens 4b..4b+3 (B: one dequantized value per lane, its token's),
+// the rows are four q heads, and CBSZ = 4 broadcasts A's block ABID to all 16:
+// A register c holds q[head l % 4][16c + l / 4], so ABID = i is accumulator
+// i's dim of chunk c, and 8 registers hold four heads' q.  A lane ends with the
+// 16 accumulators of its own token and four heads, summed by the reference's
+// tree without leaving the lane.
+// What bounds it: issue.  Per 64 tokens and four heads 128 MFMAs of 8.9 cycles
+// and 128 dequantizations of about 8 (a conversion takes 4.4 cycles, an FMA of
+// vector operands 2.8); with the q values as scalar operands of vector FMAs
+// (4.3 cycles each) the same took 3,400 cycles instead of 2,400, and waited
+// for scalar loads.  Per K-score and V-sum call of a layer: 32Q/8KV d128 at
+// 30011 tokens 17.3 against 21.2 us, 64Q/8KV at 100000 53.8 against 73.9,
+// 16Q/8KV at 20000 14.3 against 16.4, 32Q/4KV d64 at 60000 15.9 against 19.3;
+// launch-bound sizes (up to 5000 tokens) are the same.
+template <int NQ>
+struct KAcc {
+    v4f a[NQ][16];
+};
+
+// Chunk C = 4 grp + 2 nib + half of a token: its 16 values, then their products
+// with every quad of heads.
+template <int C, int D>
+__device__ __forceinline__ void k_deq(const KTok<D> &T, float *v)
 {
-    const int n_cu = cu_count();
-    const int want = (kKsBlocksPerCU * n_cu + n_kv - 1) / n_kv;
-    return want < n_sl ? want : n_sl;
+    constexpr int grp = C / 4, nib = (C >> 1) & 1, half = C & 1;
+    const uint4 r = T.raw[grp * 2 + half];
+    const uint32_t w4[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int wd = 0; wd < 4; wd++) {
+        const uint32_t n = (nib ? w4[wd] >> 4 : w4[wd]) & 0x0f0f0f0fu;
+        v[4 * wd + 0] = ubyte_f32<0>(n);
+        v[4 * wd + 1] = ubyte_f32<1>(n);
+        v[4 * wd + 2] = ubyte_f32<2>(n);
+        v[4 * wd + 3] = ubyte_f32<3>(n);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i] = fmaf(v[i], T.sc[grp], T.bi[grp]);
 }
 
-// Parts of a group's q heads, one per block (gridDim.z): where the slices
-// alone leave the chip's resident blocks unfilled (short contexts, few kv
-// heads), the largest divisor of qpk that still fits, so each lane dots
-// fewer heads (each part dequantizes its tokens again, from L2).  32Q/4KV
-// d64 at 4096 tokens: 8 parts, 512 blocks instead of 64.
-int k_head_parts(int qpk, int blocks, int n_kv)
+template <int C, int I, int D, int NQ>
+__device__ __forceinline__ void k_macs(KAcc<NQ> &acc, const float (*A)[D / 16], const float *v)
 {
-    const int64_t room = (int64_t)kKsBlocksPerCU * cu_count();
-    int hp = 1;
-    for (int d = 2; d <= qpk; d++)
-        if (qpk % d == 0 && (int64_t)n_kv * blocks * d <= room) hp = d;
-    return hp;
+    if constexpr (I < 16) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++)
+            acc.a[q][I] = __builtin_amdgcn_mfma_f32_4x4x1f32(
+                A[q][C], v[I], C == 0 ? v4f{0.0f, 0.0f, 0.0f, 0.0f} : acc.a[q][I], 4, I, 0);
+        k_macs<C, I + 1, D, NQ>(acc, A, v);
+    }
+}
+
+// The fences keep a chunk's MFMAs in one run: matrix and vector instructions of
+// a SIMD do not overlap, and each change between them costs about 5 cycles (a
+// 4x4x1 takes 8.9 cycles; one with two vector FMAs 14.0 in runs of 16, 18.9
+// taken in turn).
+template <int C, int D, int NQ>
+__device__ __forceinline__ void k_chunks(KAcc<NQ> &acc, const float (*A)[D / 16],
+                                         const KTok<D> &T)
+{
+    if constexpr (C < D / 16) {
+        float v[16];
+        k_deq<C, D>(T, v);
+        __builtin_amdgcn_sched_barrier(0);
+        k_macs<C, 0, D, NQ>(acc, A, v);
+        __builtin_amdgcn_sched_barrier(0);
+        k_chunks<C + 1, D, NQ>(acc, A, T);
+    }
+}
+
+// Block (x, kv head, z): the 256-token slices x, x + gridDim.x, ... (one token
+// per lane, the next slice's loads in flight while one is consumed), q heads
+// h_first + 4 NQ z and the 4 NQ - 1 after it of the kv head's qpk.
+template <int D, int NQ>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void k_score_mfma_kernel(
+    const uint8_t *__restrict__ kw, const float *__restrict__ ks,
+    const float *__restrict__ kb, int64_t gph, int L,
+    const float *__restrict__ q, int qpk, int h_first, float *__restrict__ scores, float rs)
+{
+    constexpr int NC = D / 16;
+    const int kvh = blockIdx.y;
+    const int n_sl = (L + 255) / 256;
+    const int64_t hb = (int64_t)kvh * gph;        // the kv head's first group
+    const uint8_t *hw = kw + hb * 32;
+    const float *hs = ks + hb, *hbi = kb + hb;
+    const int lane = threadIdx.x & 63;
+    const int h0 = h_first + 4 * NQ * (int)blockIdx.z;
+    float A[NQ][NC];
+#pragma unroll
+    for (int n = 0; n < NQ; n++) {
+        // rows past the group repeat its last head and are not stored
+        const int h = min(h0 + 4 * n + (lane & 3), qpk - 1);
+        const float *qh = q + ((int64_t)kvh * qpk + h) * D + (lane >> 2);
+#pragma unroll
+        for (int c = 0; c < NC; c++) A[n][c] = qh[16 * c];
+    }
+
+    auto compute = [&](const KTok<D> &T, int sl) {
+        KAcc<NQ> acc;
+        k_chunks<0, D, NQ>(acc, A, T);
+        const int t = sl * 256 + threadIdx.x;
+        if (t < L) {
+#pragma unroll
+            for (int n = 0; n < NQ; n++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int h = h0 + 4 * n + r;
+                    if (h >= qpk) break;
+                    float a[16];
+#pragma unroll
+                    for (int i = 0; i < 16; i++) a[i] = acc.a[n][i][r];
+                    scores[((int64_t)kvh * qpk + h) * L + t] = __fmul_rn(reduce16(a), rs);
+                }
+        }
+    };
+
+    // as k_score_mha_kernel
+    const int G = gridDim.x;
+    KTok<D> buf[kKsBufs];
+    int sl = blockIdx.x;
+#pragma unroll
+    for (int i = 0; i < kKsBufs - 1; i++) k_load<D>(hw, hs, hbi, L, sl + i * G, buf[i]);
+    for (;;) {
+#pragma unroll
+        for (int j = 0; j < kKsBufs; j++) {
+            k_load<D>(hw, hs, hbi, L, sl + (kKsBufs - 1) * G, buf[(j + kKsBufs - 1) % kKsBufs]);
+            compute(buf[j], sl);
+            sl += G;
+            if (sl >= n_sl) return;
+        }
+    }
+}
+
+// Blocks per row (n_rows rows of n_sl slices): per_cu blocks per CU over the
+// chip, at most one per slice.
+int k_blocks(int n_sl, int64_t n_rows, int per_cu)
+{
+    const int want = (int)((per_cu * cu_count() + n_rows - 1) / n_rows);
+    return want < n_sl ? want : n_sl;
 }
 
 }  // namespace
@@ -372,20 +427,40 @@ extern "C" int eakvd_k_score(const eakvd_geom *g, const uint8_t *base,
     const hipStream_t st = (hipStream_t)stream;
     const int qpk = n_q / n_kv;
     const float rs = 1.0f / sqrtf((float)g->head_dim);
-    const int kb = k_blocks(ceil_div_i(seq_len, 256), n_kv);
-    if (qpk == 1 && (int64_t)n_kv * kb < (int64_t)kKsBlocksPerCU * cu_count()) {
-        // MHA on a grid of 256-token slices that leaves the chip unfilled:
-        // four lanes per token, 64-token slices
-        const dim3 grid((unsigned)k_blocks(ceil_div_i(seq_len, 64), n_kv), (unsigned)n_kv);
+    const int n_sl = ceil_div_i(seq_len, 256);
+    if (qpk > 1) {
+        // one quad of q heads per wave (3 blocks of the kernel fit a CU) while
+        // every slice of every quad is resident at once, else two (2 blocks),
+        // which dequantize each token once for both
+        const int quads = (qpk + 3) / 4;
+        const int nq = quads > 1 && (int64_t)n_sl * n_kv * quads > 3 * (int64_t)cu_count() ? 2 : 1;
+        const int parts = (quads + nq - 1) / nq;
+        const int gx = k_blocks(n_sl, (int64_t)n_kv * parts, nq == 1 ? 3 : 2);
+        auto kern = g->head_dim == 64
+                        ? (nq == 1 ? k_score_mfma_kernel<64, 1> : k_score_mfma_kernel<64, 2>)
+                        : (nq == 1 ? k_score_mfma_kernel<128, 1> : k_score_mfma_kernel<128, 2>);
+        // one launch, but for more parts than a grid's z holds
+        for (int z0 = 0; z0 < parts; z0 += 65535) {
+            const int z = parts - z0 < 65535 ? parts - z0 : 65535;
+            hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)n_kv, (unsigned)z), dim3(256), 0,
+                               st, p.w, p.s, p.b, g->gph, seq_len, q, qpk, 4 * nq * z0, scores,
+                               rs);
+        }
+        return (int)hipGetLastError();
+    }
+    const int kb = k_blocks(n_sl, n_kv, kKsBlocksPerCU);
+    if ((int64_t)n_kv * kb < (int64_t)kKsBlocksPerCU * cu_count()) {
+        // a grid of 256-token slices that leaves the chip unfilled: four
+        // lanes per token, 64-token slices
+        const dim3 grid((unsigned)k_blocks(ceil_div_i(seq_len, 64), n_kv, kKsBlocksPerCU),
+                        (unsigned)n_kv);
         auto kern = g->head_dim == 64 ? k_score_mha4_kernel<64> : k_score_mha4_kernel<128>;
         hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, p.w, p.s, p.b, g->gph, seq_len, q,
                            scores, rs);
         return (int)hipGetLastError();
     }
-    const dim3 grid((unsigned)kb, (unsigned)n_kv, (unsigned)k_head_parts(qpk, kb, n_kv));
-    auto kern = g->head_dim == 64 ? (qpk == 1 ? k_score_mha_kernel<64> : k_score_kernel<64>)
-                                  : (qpk == 1 ? k_score_mha_kernel<128> : k_score_kernel<128>);
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, p.w, p.s, p.b, g->gph, seq_len, q, qpk,
-                       scores, rs);
+    auto kern = g->head_dim == 64 ? k_score_mha_kernel<64> : k_score_mha_kernel<128>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)kb, (unsigned)n_kv), dim3(256), 0, st, p.w, p.s, p.b,
+                       g->gph, seq_len, q, scores, rs);
     return (int)hipGetLastError();
 }
