@@ -78,9 +78,10 @@ void eakv_attention_scores(const eakv_cache_t *cc, const float *queries,
         float *dq = (float *)c->work;
         float *ds = (float *)((char *)c->work + align256(qb));
         eakvi_bounce_begin(c, qb, sb, &bo);
-        int e = eakvi_bounce_in(&bo, dq, queries, qb, st);
-        if (!e) e = eakvd_k_score(&c->geom, c->dev, layer, c->seq_len, dq, n_q,
-                                  n_kv, ds, st);
+        const void *kq;
+        int e = eakvi_bounce_in(&bo, dq, queries, qb, 0, st, &kq);
+        if (!e) e = eakvd_k_score(&c->geom, c->dev, layer, c->seq_len, kq, n_q,
+                                  n_kv, eakvi_bounce_dst(&bo, ds), st);
         if (!e) e = eakvi_bounce_out(&bo, scores_out, ds, sb, st);
         if (e) rc = eakvi_hip_fail(e, "attention_scores");
     }
@@ -146,9 +147,10 @@ void eakv_attention_output(const eakv_cache_t *cc, const float *weights,
         float *dout = (float *)((char *)c->work + align256(wb));
         void *part = (char *)c->work + align256(wb) + align256(ob);
         eakvi_bounce_begin(c, wb, ob, &bo);
-        int e = eakvi_bounce_in(&bo, dw, weights, wb, st);
-        if (!e) e = eakvd_v_sum(&c->geom, c->dev, layer, c->seq_len, dw, n_q,
-                                n_kv, dout, part, st);
+        const void *kw;
+        int e = eakvi_bounce_in(&bo, dw, weights, wb, 1, st, &kw);
+        if (!e) e = eakvd_v_sum(&c->geom, c->dev, layer, c->seq_len, kw, n_q,
+                                n_kv, eakvi_bounce_dst(&bo, dout), part, st);
         if (!e) e = eakvi_bounce_out(&bo, output_out, dout, ob, st);
         if (e) rc = eakvi_hip_fail(e, "attention_output");
     }
@@ -251,8 +253,9 @@ int eakv_attention_fused(const eakv_cache_t *cc, const float *queries,
         float *dq = (float *)c->work;
         float *dout = (float *)((char *)c->work + io);
         eakvi_bounce_begin(c, qb, qb, &bo);
-        int e = eakvi_bounce_in(&bo, dq, queries, qb, st);
-        if (!e) e = fused_launch(&c, 1, layer, dq, n_q, n_kv, dout, st);
+        const void *kq;
+        int e = eakvi_bounce_in(&bo, dq, queries, qb, 0, st, &kq);
+        if (!e) e = fused_launch(&c, 1, layer, kq, n_q, n_kv, eakvi_bounce_dst(&bo, dout), st);
         if (!e) e = eakvi_bounce_out(&bo, output_out, dout, qb, st);
         if (e) rc = eakvi_hip_fail(e, "attention_fused");
     }

@@ -166,14 +166,14 @@ int eakvi_pinned(eakv_cache_t *c, size_t n, void **p)
 }
 
 /* Inputs and results of a synchronous host-pointer call, up to kPinMax
- * bytes in all, travel through the cache's pinned host scratch: the input
- * is copied in and sent from there, the result lands there and is copied out
- * after the call's wait.  The runtime's own staging of pageable memory costs
- * more per copy (8 heads, d=128, one layer: the host-pointer V-sum
- * 27.2-27.3 against 34.8-35.0 us per call at 2048 tokens and 36.1-36.2
- * against 45.1-45.2 at 8192; the K-score 37.1-37.5 against 39.4-39.6 at
- * 8192).  Larger buffers, or no pinned memory, go from and to pageable
- * memory directly. */
+ * bytes in all, travel through the cache's pinned host scratch, which the
+ * kernels read and write in place: a copy enqueued on the stream costs 5 to 8 us,
+ * more than these calls' kernels.  One layer's step of two one-token appends,
+ * scores and output: 8Q/8KV d128 at 2048 tokens 72 us (91 with the copies), at
+ * 16384 108 (129); 64Q/8KV at 77 tokens 72 (101); 32Q/8KV at 12000, where the
+ * link's time for 3 MB counts, 216 (228).
+ * Larger buffers, or no pinned memory, are copied from and to pageable memory
+ * by the runtime. */
 #define kPinMax ((size_t)4 << 20)
 
 void eakvi_bounce_begin(eakv_cache_t *c, size_t in_b, size_t out_b, eakvi_bounce *bo)
@@ -184,18 +184,28 @@ void eakvi_bounce_begin(eakv_cache_t *c, size_t in_b, size_t out_b, eakvi_bounce
                   ? (char *)p : NULL;
 }
 
-int eakvi_bounce_in(const eakvi_bounce *bo, void *d_dst, const void *src, size_t n, void *st)
+int eakvi_bounce_in(const eakvi_bounce *bo, void *d_dst, const void *src, size_t n, int once,
+                    void *st, const void **k_src)
 {
+    *k_src = d_dst;
     if (!n) return 0;
     if (!bo->pin) return eakvd_memcpy_h2d_async(d_dst, src, n, st);
     memcpy(bo->pin, src, n);
-    return eakvd_memcpy_h2d_async(d_dst, bo->pin, n, st);
+    if (once) {
+        *k_src = bo->pin;
+        return 0;
+    }
+    return eakvd_copy_in(d_dst, bo->pin, n, st);
+}
+
+void *eakvi_bounce_dst(const eakvi_bounce *bo, void *d_dst)
+{
+    return bo->pin ? bo->pin + bo->out_off : d_dst;
 }
 
 int eakvi_bounce_out(const eakvi_bounce *bo, void *dst, const void *d_src, size_t n, void *st)
 {
-    if (!n) return 0;
-    return eakvd_memcpy_d2h_async(bo->pin ? bo->pin + bo->out_off : dst, d_src, n, st);
+    return n && !bo->pin ? eakvd_memcpy_d2h_async(dst, d_src, n, st) : 0;
 }
 
 void eakvi_bounce_end(const eakvi_bounce *bo, int rc, void *dst, size_t n)
@@ -450,14 +460,15 @@ int eakv_cache_append(eakv_cache_t *c, const float *data, int layer,
     rc = eakvi_host_begin(c);
     if (rc == EAKV_OK) rc = eakvi_work_begin(c, st, bytes);
     const int began = rc == EAKV_OK;
+    const void *src = NULL;
     if (rc == EAKV_OK) {
         eakvi_bounce bo;
         eakvi_bounce_begin(c, bytes, 0, &bo);
-        int e = eakvi_bounce_in(&bo, c->work, data, bytes, st);
+        int e = eakvi_bounce_in(&bo, c->work, data, bytes, 1, st, &src);
         if (e) rc = eakvi_hip_fail(e, "append H2D");
     }
     if (rc == EAKV_OK)
-        rc = quant_rows(c, (const float *)c->work, row_elems,
+        rc = quant_rows(c, (const float *)src, row_elems,
                         layer * 2 + kv_idx, 1, n_tokens, c->seq_len, st);
     rc = eakvi_host_end(c, rc, began, "append");
     eakvi_leave(prev);

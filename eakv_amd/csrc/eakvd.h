@@ -73,6 +73,9 @@ int  eakvd_stream_wait_event(void *s, void *e);
 int  eakvd_memset_async(void *p, int v, size_t n, void *s);
 int  eakvd_memcpy_h2d_async(void *dst, const void *src, size_t n, void *s);
 int  eakvd_memcpy_d2h_async(void *dst, const void *src, size_t n, void *s);
+/* n bytes (a multiple of 4) of pinned host memory to device memory by a small
+ * kernel: 16-byte aligned src and dst */
+int  eakvd_copy_in(void *dst, const void *src, size_t n, void *s);
 int  eakvd_memcpy_d2d_async(void *dst, const void *src, size_t n, void *s);
 const char *eakvd_error_string(int err);
 

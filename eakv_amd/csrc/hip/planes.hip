@@ -104,7 +104,27 @@ __global__ __launch_bounds__(256) void validate_kernel(const uint8_t *__restrict
     }
 }
 
+// Small inputs from pinned host memory (every byte crosses the link once; the
+// kernels that follow read them from device memory, many times).
+__global__ __launch_bounds__(256) void copy_in_kernel(float *__restrict__ dst,
+                                                      const float *__restrict__ src, int64_t n)
+{
+    const int64_t n4 = n / 4, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n4) reinterpret_cast<float4 *>(dst)[i] = reinterpret_cast<const float4 *>(src)[i];
+    else if (i < n4 + n % 4) dst[3 * n4 + i] = src[3 * n4 + i];
+}
+
 }  // namespace
+
+extern "C" int eakvd_copy_in(void *dst, const void *src, size_t n, void *stream)
+{
+    const int64_t f = (int64_t)(n / 4);
+    if (f <= 0) return 0;
+    const int64_t threads = f / 4 + f % 4;
+    hipLaunchKernelGGL(copy_in_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, (float *)dst, (const float *)src, f);
+    return (int)hipGetLastError();
+}
 
 extern "C" int eakvd_dequantize(const eakvd_geom *g, const uint8_t *base, int layer, int kv,
                                 int64_t g0, int64_t n, float *out, void *stream)

@@ -86,24 +86,30 @@ void *eakvi_batch_stream(eakv_cache_t *const *caches, int n, void *s);
 int  eakvi_host_begin(eakv_cache_t *c);
 int  eakvi_host_end(eakv_cache_t *c, int rc, int used_work, const char *what);
 
-/* The cache's pinned host scratch, at least n bytes (grown on demand; the
- * device's copies from and into pinned memory skip the runtime's staging of
- * pageable memory).  Used between eakvi_host_begin and eakvi_host_end only.
+/* The cache's pinned host scratch, at least n bytes (grown on demand; kernels
+ * read and write it in place).  Used between eakvi_host_begin and
+ * eakvi_host_end only.
  * Returns 0 or the HIP error of the allocation (the error text untouched). */
 int  eakvi_pinned(eakv_cache_t *c, size_t n, void **p);
 
 /* A host-pointer call's input and result through the pinned scratch when
- * they fit (pin NULL: pageable copies).  begin reserves in_b + out_b bytes;
- * in and out enqueue the copies on st; end copies the result out once the
- * call's wait has succeeded (rc). */
+ * they fit (pin NULL: pageable copies to and from device memory).  begin
+ * reserves in_b + out_b bytes.  in: *k_src is where the kernels read the n
+ * input bytes; an input read once stays in the scratch (`once`), one that many
+ * blocks read is taken to d_dst by a small kernel.  dst: where the kernels
+ * write the result, given its device place.  out enqueues the copy back where
+ * there is one; end copies the result out once the call's wait has succeeded
+ * (rc). */
 typedef struct {
     char  *pin;
     size_t out_off;
 } eakvi_bounce;
-void eakvi_bounce_begin(eakv_cache_t *c, size_t in_b, size_t out_b, eakvi_bounce *bo);
-int  eakvi_bounce_in(const eakvi_bounce *bo, void *d_dst, const void *src, size_t n, void *st);
-int  eakvi_bounce_out(const eakvi_bounce *bo, void *dst, const void *d_src, size_t n,
-                      void *st);
+void  eakvi_bounce_begin(eakv_cache_t *c, size_t in_b, size_t out_b, eakvi_bounce *bo);
+int   eakvi_bounce_in(const eakvi_bounce *bo, void *d_dst, const void *src, size_t n, int once,
+                      void *st, const void **k_src);
+void *eakvi_bounce_dst(const eakvi_bounce *bo, void *d_dst);
+int   eakvi_bounce_out(const eakvi_bounce *bo, void *dst, const void *d_src, size_t n,
+                       void *st);
 void eakvi_bounce_end(const eakvi_bounce *bo, int rc, void *dst, size_t n);
 
 #endif
