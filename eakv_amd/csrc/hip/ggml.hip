@@ -4,6 +4,8 @@
 // f32 vectors (reference src/ggml_type.c:21-242).  Where the reference's
 // AVX-512 and scalar paths differ, these follow the AVX-512 path (fused
 // d*n + m, 16 lane accumulators reduced by the 16-lane tree).
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -147,6 +149,106 @@ __global__ __launch_bounds__(256) void ggml_vec_dot_kernel(int nb, float *s, siz
     }
 }
 
+// The same rows dotted with one vector (a matrix times a vector): y sits in LDS,
+// and a row takes LPR lanes of A = 16 / LPR accumulators, so a lane loads A bytes
+// of each half block at once; a batch of blocks is in flight while one is
+// computed.  The tree of reduce16 is taken across the row's lanes, lane 0
+// adding in the tree's order.  The vector
+// kernel above is bound by its single-byte loads and by issue: 65,536 rows of
+// 4096 75 us against 32 here (168 MB: 5.2 TB/s), 8192 of 4096 12.9 against 9.7,
+// 4096 of 14336 44.2 against 27.3.
+template <int LPR>
+struct DotBlk {
+    static constexpr int A = 16 / LPR;
+    static constexpr int U = 4;                     // blocks per batch
+    using Q = std::conditional_t<A == 4, uint32_t, std::conditional_t<A == 2, uint16_t, uint8_t>>;
+    Q q0[U], q1[U];
+    float d[U], m[U];
+};
+
+template <int LPR>
+__global__ __launch_bounds__(256) void ggml_mat_vec_kernel(int nb, float *s, size_t bs,
+                                                           const uint8_t *vx, size_t bx,
+                                                           const float *y, int nrc)
+{
+    using B = DotBlk<LPR>;
+    constexpr int A = B::A, U = B::U;
+    extern __shared__ __attribute__((aligned(16))) float yl[];
+    const int j = threadIdx.x % LPR;
+    const int64_t r = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+    // rows past the last repeat it and are not stored
+    const uint8_t *x = vx + (r < nrc ? r : nrc - 1) * bx;
+    auto load = [&](B &b, int i0) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint8_t *blk = x + (int64_t)min(i0 + u, nb - 1) * 40;
+            b.q0[u] = *reinterpret_cast<const typename B::Q *>(blk + A * j);
+            b.q1[u] = *reinterpret_cast<const typename B::Q *>(blk + 16 + A * j);
+            b.d[u] = *reinterpret_cast<const float *>(blk + 32);
+            b.m[u] = *reinterpret_cast<const float *>(blk + 36);
+        }
+    };
+    B b0, b1;
+    load(b0, 0);
+#pragma unroll 4
+    for (int i = threadIdx.x; i < nb * 64; i += 256) yl[i] = y[i];
+    __syncthreads();
+    float a[A];
+#pragma unroll
+    for (int k = 0; k < A; k++) a[k] = 0.0f;
+    using Y = std::conditional_t<A == 4, float4, std::conditional_t<A == 2, float2, float>>;
+    auto dot1 = [&](uint32_t q, float d, float m, const float *yv) {
+        const uint32_t lo = q & 0x0f0f0f0fu, hi = (q >> 4) & 0x0f0f0f0fu;
+        float yl4[A], yh4[A];
+        *reinterpret_cast<Y *>(yl4) = *reinterpret_cast<const Y *>(yv);
+        *reinterpret_cast<Y *>(yh4) = *reinterpret_cast<const Y *>(yv + 32);
+        auto mac = [&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            if constexpr (k < A) {
+                a[k] = fmaf(fmaf(ubyte_f32<k>(lo), d, m), yl4[k], a[k]);
+                a[k] = fmaf(fmaf(ubyte_f32<k>(hi), d, m), yh4[k], a[k]);
+            }
+        };
+        mac(std::integral_constant<int, 0>{});
+        mac(std::integral_constant<int, 1>{});
+        mac(std::integral_constant<int, 2>{});
+        mac(std::integral_constant<int, 3>{});
+    };
+    auto dot = [&](const B &b, int i0) {
+        const float *yv = yl + i0 * 64 + A * j;
+        if (i0 + U <= nb) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                dot1(b.q0[u], b.d[u], b.m[u], yv + 64 * u);
+                dot1(b.q1[u], b.d[u], b.m[u], yv + 64 * u + 16);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (i0 + u < nb) {
+                    dot1(b.q0[u], b.d[u], b.m[u], yv + 64 * u);
+                    dot1(b.q1[u], b.d[u], b.m[u], yv + 64 * u + 16);
+                }
+        }
+    };
+    for (int i0 = 0; i0 < nb; i0 += 2 * U) {
+        load(b1, i0 + U);
+        dot(b0, i0);
+        load(b0, i0 + 2 * U);
+        dot(b1, i0 + U);
+    }
+    // accumulator A j + k of lane j; v8[i] = a[i] + a[i + 8], then + 4, + 2, + 1
+#pragma unroll
+    for (int o = LPR / 2; o >= 1; o >>= 1)
+#pragma unroll
+        for (int k = 0; k < A; k++) a[k] = __fadd_rn(a[k], __shfl_xor(a[k], o, LPR));
+    float t = a[0];
+    if constexpr (A == 4) t = __fadd_rn(__fadd_rn(a[0], a[2]), __fadd_rn(a[1], a[3]));
+    if constexpr (A == 2) t = __fadd_rn(a[0], a[1]);
+    if (j == 0 && r < nrc)
+        *reinterpret_cast<float *>(reinterpret_cast<char *>(s) + r * bs) = t;
+}
+
 // One pass over the threads up to 65,535 blocks (the dequantizer at 65,536
 // rows of 4096: 184.2-184.5 against 199.7-200.3 us per call with at most
 // 8192 blocks and eight blocks' work per lane)
@@ -192,6 +294,21 @@ extern "C" int eakvd_ggml_vec_dot(int n, float *s, size_t bs, const void *vx, si
                                   const void *vy, size_t by, int nrc, void *stream)
 {
     if (nrc <= 0) return 0;
+    // One vector for all rows, whole in LDS (up to 64 KB): from 2048 rows on,
+    // where the copy of y into LDS is made up for (100 rows of 11008: 18.3
+    // against 18.5 us), with as few lanes a row as still fill the chip's SIMDs
+    // about twice (8192 rows of 4096: 9.7 us with 16 lanes, 10.4 with 8, 13.4
+    // with 4; 32768 of 1024: 10.1, 7.7, 6.7).
+    if (by == 0 && nrc >= 2048 && n >= 64 && n <= 16384) {
+        const int lpr = nrc >= 32768 ? 4 : nrc >= 16384 ? 8 : 16;
+        auto kern = lpr == 4 ? ggml_mat_vec_kernel<4> : lpr == 8 ? ggml_mat_vec_kernel<8>
+                                                                 : ggml_mat_vec_kernel<16>;
+        const int64_t blocks = ((int64_t)nrc * lpr + 255) / 256;
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), (size_t)(n / 64) * 256,
+                           (hipStream_t)stream, n / 64, s, bs, (const uint8_t *)vx, bx,
+                           (const float *)vy, nrc);
+        return (int)hipGetLastError();
+    }
     hipLaunchKernelGGL(ggml_vec_dot_kernel, dim3(grid_for((int64_t)nrc * 16)), dim3(256), 0,
                        (hipStream_t)stream, n / 64, s, bs, (const uint8_t *)vx, bx,
                        (const uint8_t *)vy, by, nrc);
