@@ -427,9 +427,17 @@ struct WaveState {
 // the merge launch the same call would make, in the same order, so both give
 // the same bits: merge_kernel, and vsum_merge_kernel in V-sum mode.  Loads:
 // the (m, l) pair of every (head, chunk) once per block into LDS (one 8-byte
-// device-scope load each), and per thread the o values of kInBatch chunks
+// device-scope load each), and per thread the o values of NB chunks
 // (one 4- or 8-byte device-scope load each), all issued before the barrier:
-// one round trip.
+// one round trip.  The lanes' offsets are known before the block counts itself
+// (MergeOffs), so nothing but the loads follows the count; NB is 8 or 16, the
+// entries past the last chunk weighing 0.
+// What bounds it is the chain of one block: with the divisions, 64-bit
+// addresses and selects over 16 entries behind the count, the merge took 3,000
+// of a 12,400-cycle call.  Without, and with a unit's only chunk written
+// directly (one_chunk), a layer takes: 32Q/8KV d128 at 100 tokens 6.1 against
+// 7.1 us, 8Q/8KV at 2048 6.3 against 6.7, 24 x 32Q/32KV at 600 tokens 16.7
+// against 20, 8 x 32Q/8KV at 32768 55.2 against 56.0.
 // (A first form had every thread load m, l and o of kInBatch clamped chunks
 // for each of its outputs, 96 loads per thread; its merge cost about 3 us of
 // an 8 x 32Q/8KV call at 32767 tokens.)
@@ -439,77 +447,87 @@ constexpr int kInParts = 8;     // vsum_merge_kernel's parts
 // pu: the partials of the unit's first q head (head h, chunk c at
 // (h * nb + c) * (D + 2): m, l, o[D]); stage: LDS, 2 * kInBatch floats per
 // head; G q heads; outputs ou[G][D]; P adjacent outputs per thread (1 where
-// G * D <= nthreads, else 2).  Every thread of the block calls it (it holds
-// a barrier).
-template <int D, bool VS, int P>
-__device__ __forceinline__ void merge_unit_p(const float *pu, int nb, int n_chunks, int G,
-                                             float *stage, float *ou, int tid)
+// G * D <= the block's threads, else 2).
+struct MergeOffs {
+    uint32_t o;         // bytes from pu to the thread's o of chunk 0
+    uint32_t ml;        // to its (m, l) pair
+    int out;            // its output, -1: none
+};
+
+template <int D>
+__device__ __forceinline__ MergeOffs merge_offs(int nb, int n_chunks, int G, int tid,
+                                                int nthreads)
 {
-    const bool has = P * tid < G * D;
-    const int h = has ? P * tid / D : 0, dim = P * tid % D;
-    const float *ph = pu + (int64_t)h * nb * (D + 2) + 2 + dim;
-    // the (m, l) pair of (head, chunk) k = tid (G * n_chunks <= nthreads),
-    // then the o values: unconditional, clamped to the last chunk, no branch
-    // between the loads (entries past the last chunk hold its values); the
-    // pair goes to LDS once its load is in, the o loads still in flight
-    const bool stg = tid < G * n_chunks;
-    const int sh = stg ? tid / n_chunks : 0, sc = stg ? tid % n_chunks : 0;
-    const float2 ml = ld_dev2(pu + ((int64_t)sh * nb + sc) * (D + 2));
-    float ov[kInBatch][P];
+    const int P = G * D <= nthreads ? 1 : 2;
+    const int NB = n_chunks <= 8 ? 8 : kInBatch;
+    const int i = P * tid, h = i / D, sh = tid / NB, sc = tid % NB;
+    MergeOffs m;
+    m.out = i < G * D ? i : -1;
+    m.o = (uint32_t)(((i < G * D ? h : 0) * nb * (D + 2) + 2 + i % D) * 4);
+    m.ml = (uint32_t)(((sh < G ? sh : 0) * nb + (sc < n_chunks ? sc : 0)) * (D + 2) * 4);
+    asm volatile("" : "+v"(m.o), "+v"(m.ml), "+v"(m.out));
+    return m;
+}
+
+// the float at byte offset o of a uniform address
+__device__ __forceinline__ const float *at_bytes(const float *p, uint32_t o)
+{
+    return reinterpret_cast<const float *>(reinterpret_cast<const char *>(p) + o);
+}
+
+template <int D, bool VS, int P, int NB>
+__device__ __forceinline__ void merge_unit_p(const float *pu, const MergeOffs &mo,
+                                             int n_chunks, int G, float *stage, float *ou, int tid)
+{
+    const float2 ml = ld_dev2(at_bytes(pu, mo.ml));
+    float ov[NB][P];
 #pragma unroll
-    for (int j = 0; j < kInBatch; j++) {
-        const float *pj = ph + min(j, n_chunks - 1) * (D + 2);
+    for (int j = 0; j < NB; j++) {
+        // unconditional, clamped to the last chunk
+        const float *pj = pu + min(j, n_chunks - 1) * (D + 2);
         if constexpr (P == 2) {
-            const float2 v = ld_dev2(pj);
+            const float2 v = ld_dev2(at_bytes(pj, mo.o));
             ov[j][0] = v.x;
             ov[j][1] = v.y;
         } else {
-            ov[j][0] = ld_dev(pj);
+            ov[j][0] = ld_dev(at_bytes(pj, mo.o));
         }
     }
-    if (stg) {
-        stage[sh * 2 * kInBatch + sc] = ml.x;
-        stage[sh * 2 * kInBatch + kInBatch + sc] = ml.y;
+    const int sh = tid / NB, sc = tid % NB;
+    if (sh < G) {
+        stage[sh * 2 * NB + sc] = sc < n_chunks ? ml.x : -INFINITY;
+        stage[sh * 2 * NB + NB + sc] = sc < n_chunks ? ml.y : 0.0f;
     }
     __syncthreads();
-    if (!has) return;
+    if (mo.out < 0) return;
     // every staged (m, l) of the head into registers at once (16-byte LDS
-    // reads; entries past the last chunk are not used or are replaced by
-    // the last chunk's l), so the selects below need no LDS round trips
-    const float4 *m4 = reinterpret_cast<const float4 *>(stage + h * 2 * kInBatch);
-    float mv[kInBatch], lv[kInBatch];
+    // reads)
+    const float4 *m4 = reinterpret_cast<const float4 *>(stage + mo.out / D * 2 * NB);
+    float mv[NB], lv[NB];
 #pragma unroll
-    for (int q = 0; q < kInBatch / 4; q++) {
-        const float4 a = m4[q], b = m4[kInBatch / 4 + q];
+    for (int q = 0; q < NB / 4; q++) {
+        const float4 a = m4[q], b = m4[NB / 4 + q];
         mv[4 * q] = a.x; mv[4 * q + 1] = a.y; mv[4 * q + 2] = a.z; mv[4 * q + 3] = a.w;
         lv[4 * q] = b.x; lv[4 * q + 1] = b.y; lv[4 * q + 2] = b.z; lv[4 * q + 3] = b.w;
     }
-    float r[P];
+    float res[P];
     if constexpr (!VS) {
         // softmax merge: M = max(-1e6 log2(e), m_c), l = sum l_c 2^(m_c - M),
-        // o = sum o_c 2^(m_c - M), out = o * (1/l); the batch's entries past
-        // the last chunk repeat the last chunk's l and o with weight 0
-        const float M = -1000000.0f * EAKV_LOG2E;
-        float Mn = M, lt = 0.0f, o[P];
+        // o = sum o_c 2^(m_c - M), out = o * (1/l)
+        float M = -1000000.0f * EAKV_LOG2E, lt = 0.0f, o[P];
 #pragma unroll
         for (int e = 0; e < P; e++) o[e] = 0.0f;
 #pragma unroll
-        for (int j = 0; j < kInBatch; j++) Mn = j < n_chunks ? fmaxf(Mn, mv[j]) : Mn;
-        const float f = __builtin_amdgcn_exp2f(M - Mn);
-        lt *= f;
+        for (int j = 0; j < NB; j++) M = fmaxf(M, mv[j]);
 #pragma unroll
-        for (int e = 0; e < P; e++) o[e] *= f;
-        const float llast = stage[h * 2 * kInBatch + kInBatch + n_chunks - 1];
-#pragma unroll
-        for (int j = 0; j < kInBatch; j++) {
-            const bool in = j < n_chunks;
-            const float wj = in ? __builtin_amdgcn_exp2f(mv[j] - Mn) : 0.0f;
-            lt = fmaf(in ? lv[j] : llast, wj, lt);
+        for (int j = 0; j < NB; j++) {
+            const float wj = __builtin_amdgcn_exp2f(mv[j] - M);
+            lt = fmaf(lv[j], wj, lt);
 #pragma unroll
             for (int e = 0; e < P; e++) o[e] = fmaf(ov[j][e], wj, o[e]);
         }
 #pragma unroll
-        for (int e = 0; e < P; e++) r[e] = o[e] * (1.0f / lt);
+        for (int e = 0; e < P; e++) res[e] = o[e] * (1.0f / lt);
     } else {
         // V-sum: the plain sum of o_c in 8 strided parts (chunks pt, pt + 8)
         // added in part order, NaN when a chunk's l is NaN (a non-finite
@@ -523,29 +541,48 @@ __device__ __forceinline__ void merge_unit_p(const float *pu, int nb, int n_chun
 #pragma unroll
             for (int e = 0; e < P; e++) sm[e] = 0.0f;
 #pragma unroll
-            for (int c = pt; c < kInBatch; c += kInParts) {
+            for (int c = pt; c < NB; c += kInParts) {
                 const bool in = c < n_chunks;
 #pragma unroll
                 for (int e = 0; e < P; e++) sm[e] = in ? __fadd_rn(sm[e], ov[c][e]) : sm[e];
-                bad = in ? bad + lv[c] : bad;     // 0, or NaN after a non-finite weight
+                bad += lv[c];                     // 0, or NaN after a non-finite weight
             }
 #pragma unroll
             for (int e = 0; e < P; e++) t[e] = pt == 0 ? sm[e] : __fadd_rn(t[e], sm[e]);
             fl = pt == 0 ? bad : fl + bad;
         }
 #pragma unroll
-        for (int e = 0; e < P; e++) r[e] = fl == fl ? t[e] : fl;
+        for (int e = 0; e < P; e++) res[e] = fl == fl ? t[e] : fl;
     }
 #pragma unroll
-    for (int e = 0; e < P; e++) ou[h * D + dim + e] = r[e];
+    for (int e = 0; e < P; e++) ou[mo.out + e] = res[e];
 }
 
+// every thread of the block calls it (it holds a barrier)
 template <int D, bool VS>
-__device__ __forceinline__ void merge_unit(const float *pu, int nb, int n_chunks, int G,
-                                           float *stage, float *ou, int tid, int nthreads)
+__device__ __forceinline__ void merge_unit(const float *pu, const MergeOffs &mo,
+                                           int n_chunks, int G, float *stage, float *ou, int tid,
+                                           int nthreads)
 {
-    if (G * D <= nthreads) merge_unit_p<D, VS, 1>(pu, nb, n_chunks, G, stage, ou, tid);
-    else merge_unit_p<D, VS, 2>(pu, nb, n_chunks, G, stage, ou, tid);
+    if (G * D <= nthreads) {
+        if (n_chunks <= 8) merge_unit_p<D, VS, 1, 8>(pu, mo, n_chunks, G, stage, ou, tid);
+        else merge_unit_p<D, VS, 1, kInBatch>(pu, mo, n_chunks, G, stage, ou, tid);
+    } else {
+        if (n_chunks <= 8) merge_unit_p<D, VS, 2, 8>(pu, mo, n_chunks, G, stage, ou, tid);
+        else merge_unit_p<D, VS, 2, kInBatch>(pu, mo, n_chunks, G, stage, ou, tid);
+    }
+}
+
+// The result of a unit's only chunk: what the merge makes of one partial.
+template <bool VS>
+__device__ __forceinline__ float one_chunk(float M, float l, float o)
+{
+    if constexpr (VS) {
+        return l == l ? __fadd_rn(0.0f, o) : l;
+    } else {
+        const float f = __builtin_amdgcn_exp2f(M - fmaxf(-1000000.0f * EAKV_LOG2E, M));
+        return fmaf(o, f, 0.0f) * (1.0f / fmaf(l, f, 0.0f));
+    }
 }
 
 // The chunks of a launch: sequence s has pre[s + 1] - pre[s] of them per
@@ -617,10 +654,9 @@ __device__ __forceinline__ void mfma_body(
                  "s"(g.block_bytes), "s"(ctr), "s"(lead_from), "s"(part), "s"(rs), "s"(out));
     const int n_tiles = (L + TT - 1) / TT;
     if (ch * NW >= n_tiles) {         // no tile for this block: no partial
-        // merged here, an empty sequence's outputs are 0 * (1/0) = NaN, as
-        // the reference's (and merge_kernel's)
+        // an empty sequence's outputs are 0 * (1/0) = NaN, as the reference's
         if constexpr (!VS)
-            if (ctr && n_tiles == 0 && ch == 0) {
+            if (n_tiles == 0 && ch == 0) {
                 const float zl = 0.0f, zo = 0.0f;
                 for (int i = threadIdx.x; i < qpk * D; i += 64 * NW)
                     out[((int64_t)s * n_q + (int64_t)kvh * qpk) * D + i] = zo * (1.0f / zl);
@@ -1253,6 +1289,9 @@ __device__ __forceinline__ void mfma_body(
 
     // ---- merge the waves into this chunk's partial, two adjacent outputs
     // of one head per thread (their scale factors computed once)
+    const int n_chunks = min(nb, (n_tiles + NW - 1) / NW);   // blocks with a tile
+    float *pu = part + ((int64_t)pre * n_q + kvh * qpk * nb) * (D + 2);
+    float *ou = out + ((int64_t)s * n_q + kvh * qpk) * D;
     for (int i2 = tid; 2 * i2 < G * D; i2 += 64 * NW) {
         const int h = 2 * i2 / D, dim = 2 * i2 % D;
         float M = -INFINITY;
@@ -1269,7 +1308,12 @@ __device__ __forceinline__ void mfma_body(
             o0 = fmaf(ov.x, f, o0);
             o1 = fmaf(ov.y, f, o1);
         }
-        float *dst = part + ((int64_t)pre * n_q + (kvh * qpk + h) * nb + ch) * (D + 2);
+        if (n_chunks == 1) {
+            *reinterpret_cast<float2 *>(ou + h * D + dim) =
+                make_float2(one_chunk<VS>(M, lt, o0), one_chunk<VS>(M, lt, o1));
+            continue;
+        }
+        float *dst = pu + (h * nb + ch) * (D + 2);
         if (ctr) {
             st_dev2(dst + 2 + dim, o0, o1);
             if (dim == 0) st_dev2(dst, M, lt);
@@ -1278,7 +1322,7 @@ __device__ __forceinline__ void mfma_body(
             if (dim == 0) *reinterpret_cast<float2 *>(dst) = make_float2(M, lt);
         }
     }
-    if (!ctr) return;
+    if (!ctr || n_chunks == 1) return;
 
     // ---- the chunk merge in this launch: every thread's
     // partial stores are complete (vmcnt 0) before the barrier, and so
@@ -1286,7 +1330,7 @@ __device__ __forceinline__ void mfma_body(
     // counts last reads the unit's partials after it, merges them into out
     // and sets the counter back to zero (no other block of the launch
     // touches it again)
-    const int n_chunks = min(nb, (n_tiles + NW - 1) / NW);   // blocks with a tile
+    const MergeOffs mo = merge_offs<D>(nb, n_chunks, G, tid, 64 * NW);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     unsigned *uc = reinterpret_cast<unsigned *>(
@@ -1300,8 +1344,7 @@ __device__ __forceinline__ void mfma_body(
     if (tid == 0) __hip_atomic_store(uc, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     static_assert(4 * HH * D / 2 <= 64 * NW && 4 * HH * kInBatch <= 64 * NW,
                   "one output pair and at most one (m, l) pair per thread");
-    merge_unit<D, VS>(part + ((int64_t)pre * n_q + kvh * qpk * nb) * (D + 2), nb, n_chunks, G,
-                      &s_lds0[0][0], out + ((int64_t)s * n_q + kvh * qpk) * D, tid, 64 * NW);
+    merge_unit<D, VS>(pu, mo, n_chunks, G, &s_lds0[0][0], ou, tid, 64 * NW);
 }
 
 // Every sequence in gridDim.x chunks: the grid is (chunk, virtual kv head,
@@ -1356,6 +1399,7 @@ __global__ __launch_bounds__(D) void merge_kernel(
     const int max_chunks = cm.pre[s + 1] - cm.pre[s];
     const int n_tiles = (bt.seq_len[s] + tt - 1) / tt;
     const int n_chunks = min(max_chunks, (n_tiles + wpb - 1) / wpb);
+    if (n_chunks <= 1) return;          // written by mfma_body
     const float *p = part + ((int64_t)cm.pre[s] * n_q + qh * max_chunks) * (D + 2);
     // The (m, l) pair and o[i] of every chunk by vector buffer loads, all
     // issued before any arithmetic: one memory round trip.  (As scalar
@@ -1413,6 +1457,7 @@ __global__ __launch_bounds__(256) void merge_parts_kernel(
     const int max_chunks = cm.pre[s + 1] - cm.pre[s];
     const int n_tiles = (bt.seq_len[s] + tt - 1) / tt;
     const int n_chunks = min(max_chunks, (n_tiles + wpb - 1) / wpb);
+    if (n_chunks <= 1) return;          // written by mfma_body
     const float *p = part + ((int64_t)cm.pre[s] * n_q + qh * max_chunks) * (D + 2);
     float M = -1000000.0f * EAKV_LOG2E, lt = 0.0f, ot = 0.0f;
     for (int c0 = pt; c0 < n_chunks; c0 += kMergeParts * kPartBatch) {
@@ -2014,7 +2059,7 @@ extern "C" int eakvd_fused(const eakvd_geom *g, const eakvd_batch *b,
             hipLaunchKernelGGL(ragged_entry(g->head_dim, hh, p.tt), dim3((unsigned)blocks),
                                dim3(64 * wpb), 0, st, *g, *b, p.cm, layer, q, n_q, p.qv, rs,
                                part, p.split, out, uc, vkv, lead_from);
-        if (uc) return (int)hipGetLastError();
+        if (uc || mc == 1) return (int)hipGetLastError();
         const int tt = p.tt;
         if (parts && g->head_dim == 64)
             hipLaunchKernelGGL(merge_parts_kernel<64>, pgrid, dim3(256), 0, st, *b, p.cm, n_q,
@@ -2095,9 +2140,10 @@ extern "C" int eakvd_v_sum_mfma(const eakvd_geom *g, const uint8_t *base, int la
     hipLaunchKernelGGL(kern, grid, dim3(64 * wpb), 0, st, *g, b, layer, w, n_q, qv, 0.0f,
                        part, split, out, uc, 0);
     if (uc) return (int)hipGetLastError();
-    // the chunks that hold a partial: blocks with a tile (see mfma_kernel)
+    // the chunks that hold a partial: blocks with a tile (see mfma_body)
     const int n_tiles = (seq_len + tt - 1) / tt;
     const int nch = min(mc, (n_tiles + wpb - 1) / wpb);
+    if (nch == 1) return (int)hipGetLastError();
     if (g->head_dim == 64)
         hipLaunchKernelGGL(vsum_merge_kernel<64>, dim3((unsigned)(n_q * 2)), dim3(256), 0, st,
                            mc, nch, part, out);

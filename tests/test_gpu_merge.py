@@ -1,0 +1,50 @@
+"""The chunk merge inside the fused launch and its V-sum form at their edges:
+one chunk (written directly), 2, 8 and 9 (both batch sizes), 16, one and two
+outputs per thread, more one-chunk units than counters, and empty sequences.
+Both entry points give the same bits; results meet the reference bar."""
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import tol_close
+from test_gpu_headline import (E, batch_call, build_batch, chan_k,  # noqa: F401
+                               compare_sequences, n_cu, say)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n_kv,n_q,n_seq,L,chunks", [
+    (8, 8, 1, 100, 1), (8, 32, 1, 128, 1), (4, 8, 1, 200, 2), (8, 32, 1, 1024, 8),
+    (8, 8, 1, 1025, 9), (8, 32, 1, 1025, 9), (4, 16, 1, 2048, 16), (32, 32, 16, 300, 1)])
+def test_merge_edges(E, d, n_kv, n_q, n_seq, L, chunks):  # noqa: F811
+    gs, os_ = build_batch(E, 0xEA4B + 800 + d + L, n_seq, n_kv, d, [L] * n_seq, L + 3, chan_k)
+    plan = E.fused_plan(gs, n_q, n_kv)
+    say("merge: plan", plan)
+    if n_cu() == 256:
+        assert plan["chunks"] == chunks
+    rng = np.random.default_rng(0xEA4B + 801 + d)
+    q = rng.standard_normal((n_seq, n_q, d), dtype=np.float32)
+    out = batch_call(E, "eakv_attention_fused_batch_device", gs, q, n_q, n_kv)
+    out_na = batch_call(E, "eakv_attention_fused_batch_device_noalloc", gs, q, n_q, n_kv)
+    assert np.array_equal(out.view(np.uint32), out_na.view(np.uint32))
+    compare_sequences(os_, q, out, n_q, n_kv, [L] * n_seq)
+    w = O.softmax_rows(os_[0].attention_scores(q[0], 0, n_q, n_kv))
+    w[0, 0] = -w[0, 0]
+    ok, err, bad = tol_close(gs[0].attention_output(w, 0, n_q, n_kv),
+                             os_[0].attention_output(w, 0, n_q, n_kv))
+    assert ok, (err, bad)
+    w[n_q - 1, 0] = np.inf
+    got = gs[0].attention_output(w, 0, n_q, n_kv)
+    assert not np.isfinite(got[n_q - 1]).any() and np.isfinite(got[:n_q - 1]).all()
+    for g in gs:
+        g.free()
+
+
+def test_empty_batch(E):  # noqa: F811
+    gs = [E.Cache(1, 2, 64, 40) for _ in range(3)]
+    q = np.ones((3, 4, 64), np.float32)
+    for fn in ("eakv_attention_fused_batch_device", "eakv_attention_fused_batch_device_noalloc"):
+        assert np.isnan(batch_call(E, fn, gs, q, 4, 2)).all()
+    for g in gs:
+        g.free()
