@@ -1752,11 +1752,19 @@ __global__ __launch_bounds__(D) void combine_kernel(
 // 11.7 -> 10.5 us and 32Q/4KV d64 at 4096 10.3 -> 9.6 us with 256-token
 // chunks, but 32Q/32KV at 8192 15.0 -> 17.5 us with them everywhere; 8Q/8KV
 // at 2048 tokens 6.86 -> 6.31 us with 128-token chunks (one tile per wave).
-int mfma_blocks_per_unit(int ml, int units, int per_cu)
+// One-quad units that fill more than half but at most three quarters of the
+// slots take two chunks each over long contexts: a third block fits a CU
+// (registers and LDS), so all are resident, where one chunk each left the CUs
+// with one or two (9 sequences of 32Q/32KV at 6000 tokens 57.5 against 64 us a
+// layer, 10 at 8000 75 against 85, 12 at 4000 44.7 against 47.2; 24 of 12Q/12KV
+// d64 at 9000 41 against 49; but 9 at 1500 21.5 against 20.2, and a third chunk
+// at 24 of 32Q/8KV 51.7 against 50.7).
+int mfma_blocks_per_unit(int ml, int units, int per_cu, int hh)
 {
     const int n_cu = cu_count();
     const int slots = n_cu * per_cu;
     int nb = units >= slots ? 1 : slots / units;
+    if (nb == 1 && hh == 1 && 4 * units <= 3 * slots && ml >= 24 * kChunkM) nb = 2;
     const int coarse = (ml + 4 * kChunkM - 1) / (4 * kChunkM);
     int fine = (ml + kChunkM - 1) / kChunkM;
     if (fine > kInBatch) fine = max(kInBatch, (ml + 2 * kChunkM - 1) / (2 * kChunkM));
@@ -1800,7 +1808,7 @@ int mfma_split_fill(int qpk, int d, int ml, int64_t units)
     const int sp = mfma_split(qpk);
     if (sp != 1 || qpk <= 4 || qpk % 2) return sp;
     const int per_cu = per_cu_of(d, 2);
-    const int64_t blocks = units * mfma_blocks_per_unit(ml, (int)units, per_cu);
+    const int64_t blocks = units * mfma_blocks_per_unit(ml, (int)units, per_cu, 2);
     return 2 * blocks < (int64_t)cu_count() * per_cu ? 2 : 1;
 }
 
@@ -1940,7 +1948,7 @@ FusedPlan fused_plan(const eakvd_geom *g, const eakvd_batch *b, int n_q, int n_k
         p.hh = p.qv <= 4 ? 1 : 2;
         const int per_cu = per_cu_of(g->head_dim, p.hh);
         p.wpb = p.hh == 1 ? kWavesH<1> : kWavesH<2>;
-        p.mc = mfma_blocks_per_unit(ml, b->n_seq * n_kv * p.split, per_cu);
+        p.mc = mfma_blocks_per_unit(ml, b->n_seq * n_kv * p.split, per_cu, p.hh);
         p.tt = tile_tokens(p.hh, ml, p.mc, p.wpb);
         bool ragged = false;
         for (int i = 1; i < b->n_seq; i++) ragged = ragged || b->seq_len[i] != b->seq_len[0];
@@ -2142,7 +2150,7 @@ extern "C" int eakvd_v_sum_mfma(const eakvd_geom *g, const uint8_t *base, int la
     const int hh = qv <= 4 ? 1 : 2;
     const int per_cu = per_cu_of(g->head_dim, hh);
     const int wpb = hh == 1 ? kWavesH<1> : kWavesH<2>;
-    const int mc = mfma_blocks_per_unit(seq_len, n_kv * split, per_cu);
+    const int mc = mfma_blocks_per_unit(seq_len, n_kv * split, per_cu, hh);
     const int tt = tile_tokens(hh, seq_len, mc, wpb);
     const dim3 grid((unsigned)mc, (unsigned)(n_kv * split), 1u);
     float *part = (float *)work;

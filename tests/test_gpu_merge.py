@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("n_kv,n_q,n_seq,L,chunks", [
     (8, 8, 1, 100, 1), (8, 32, 1, 128, 1), (4, 8, 1, 200, 2), (8, 32, 1, 1024, 8),
-    (8, 8, 1, 1025, 9), (8, 32, 1, 1025, 9), (4, 16, 1, 2048, 16), (32, 32, 16, 300, 1)])
+    (8, 8, 1, 1025, 9), (8, 32, 1, 1025, 9), (4, 16, 1, 2048, 16), (32, 32, 16, 300, 1),
+    (32, 32, 9, 3071, 1), (32, 32, 9, 3072, 2)])
 def test_merge_edges(E, d, n_kv, n_q, n_seq, L, chunks):  # noqa: F811
     gs, os_ = build_batch(E, 0xEA4B + 800 + d + L, n_seq, n_kv, d, [L] * n_seq, L + 3, chan_k)
     plan = E.fused_plan(gs, n_q, n_kv)
