@@ -6,9 +6,10 @@
 // extended per q head to GQA and d=64.  Each q head h reads kv head
 // h / (n_q/n_kv).
 //
-// Work split (flash-decoding): one block per (sequence, kv head, chunk);
-// each block writes a partial (m, l, o[D]) per q head and merge_kernel
-// combines the chunks.
+// Work split (flash-decoding): one block per (sequence, kv head, chunk), as
+// many chunks for every sequence (mfma_kernel) or, for contexts of several
+// lengths, in proportion to each (ragged_kernel); each block writes a partial
+// (m, l, o[D]) per q head and the chunks are merged.
 //
 // Two block programs:
 //
@@ -1389,8 +1390,8 @@ __global__ __launch_bounds__(64 * kWavesH<HH>, (kWavesH<HH> * kBlocksPerCUH<D, H
 // sequence): M = max(-1e6 log2(e), m_c) (the reference's max starts at
 // -1e6), l = sum l_c 2^(m_c - M), o = sum o_c 2^(m_c - M), out = o * (1/l).
 // The chunks are read kMergeBatch at a time with all loads in flight and
-// merged online across batches.  An empty sequence has no chunks:
-// 0 * (1/0) = NaN, as the reference.
+// merged online across batches.  Units of one chunk, and empty sequences, are
+// written by mfma_body.
 constexpr int kMergeBatch = 16;
 
 template <int D>
@@ -1444,8 +1445,8 @@ __global__ __launch_bounds__(D) void merge_kernel(
 // The same merge for more than kMergeBatch chunks (long contexts): a block
 // takes 32 dims of one (q head, sequence); thread (i, part) merges
 // chunks part, part + 8, ... online, kPartBatch at a time with their loads
-// in flight, and the 8 part results are merged in part order.  An empty
-// sequence has no chunks: 0 * (1/0) = NaN, as the reference.
+// in flight, and the 8 part results are merged in part order.  Units of one
+// chunk, and empty sequences, are written by mfma_body.
 constexpr int kMergeParts = 8;
 constexpr int kPartBatch = 8;
 

@@ -136,8 +136,8 @@ int eakv_attention_fused_batch_device_noalloc(eakv_cache_t *const *caches,
  * allocation-free form (noalloc != 0) makes for these caches at their
  * current seq_len and this head split, for diagnostics and tests; nothing is
  * launched.  plan (8 entries): [0] 1 for the matrix-core program, 0 for the
- * VALU program (layer blocks beyond 32-bit buffer offsets); [1] chunks per
- * (sequence, kv head) unit; [2] 1 when the chunks are merged inside the
+ * VALU program (layer blocks beyond 32-bit buffer offsets); [1] the most
+ * chunks of a (sequence, kv head) unit; [2] 1 when the chunks are merged inside the
  * launch (up to 16 chunks per unit), 0 when a merge launch follows; [3]
  * tokens per tile; [4] waves per
  * block; [5] the most tiles one wave walks; [6] quads of q heads per wave;
