@@ -432,7 +432,7 @@ struct WaveState {
 // (one 4- or 8-byte device-scope load each), all issued before the barrier:
 // one round trip.  The lanes' offsets are known before the block counts itself
 // (MergeOffs), so nothing but the loads follows the count; NB is 8 or 16, the
-// entries past the last chunk weighing 0.
+// entries past the last chunk adding nothing.
 // What bounds it is the chain of one block: with the divisions, 64-bit
 // addresses and selects over 16 entries behind the count, the merge took 3,000
 // of a 12,400-cycle call.  Without, and with a unit's only chunk written
@@ -514,7 +514,9 @@ __device__ __forceinline__ void merge_unit_p(const float *pu, const MergeOffs &m
     float res[P];
     if constexpr (!VS) {
         // softmax merge: M = max(-1e6 log2(e), m_c), l = sum l_c 2^(m_c - M),
-        // o = sum o_c 2^(m_c - M), out = o * (1/l)
+        // o = sum o_c 2^(m_c - M), out = o * (1/l).  Past the last chunk 0 of
+        // weight 0: the loaded o, the last chunk's, would add NaN where it is
+        // infinite.
         float M = -1000000.0f * EAKV_LOG2E, lt = 0.0f, o[P];
 #pragma unroll
         for (int e = 0; e < P; e++) o[e] = 0.0f;
@@ -525,10 +527,10 @@ __device__ __forceinline__ void merge_unit_p(const float *pu, const MergeOffs &m
             const float wj = __builtin_amdgcn_exp2f(mv[j] - M);
             lt = fmaf(lv[j], wj, lt);
 #pragma unroll
-            for (int e = 0; e < P; e++) o[e] = fmaf(ov[j][e], wj, o[e]);
+            for (int e = 0; e < P; e++) o[e] = fmaf(j < n_chunks ? ov[j][e] : 0.0f, wj, o[e]);
         }
 #pragma unroll
-        for (int e = 0; e < P; e++) res[e] = o[e] * (1.0f / lt);
+        for (int e = 0; e < P; e++) res[e] = __fadd_rn(o[e], 0.0f) * (1.0f / lt);
     } else {
         // V-sum: the plain sum of o_c in 8 strided parts (chunks pt, pt + 8)
         // added in part order, NaN when a chunk's l is NaN (a non-finite
@@ -1433,13 +1435,16 @@ __global__ __launch_bounds__(D) void merge_kernel(
         ot *= f;
 #pragma unroll
         for (int j = 0; j < kMergeBatch; j++) {
-            const float wj = c0 + j < n_chunks ? __builtin_amdgcn_exp2f(m[j] - Mn) : 0.0f;
-            lt = fmaf(lv[j], wj, lt);
-            ot = fmaf(ov[j], wj, ot);
+            // past the last chunk 0, as in merge_unit_p
+            const bool in = c0 + j < n_chunks;
+            const float wj = in ? __builtin_amdgcn_exp2f(m[j] - Mn) : 0.0f;
+            lt = fmaf(in ? lv[j] : 0.0f, wj, lt);
+            ot = fmaf(in ? ov[j] : 0.0f, wj, ot);
         }
         M = Mn;
     }
-    out[((int64_t)s * n_q + qh) * D + i] = ot * (1.0f / lt);
+    // + 0: the same zero whatever the number of entries past the last chunk
+    out[((int64_t)s * n_q + qh) * D + i] = __fadd_rn(ot, 0.0f) * (1.0f / lt);
 }
 
 // The same merge for more than kMergeBatch chunks (long contexts): a block
@@ -1484,10 +1489,11 @@ __global__ __launch_bounds__(256) void merge_parts_kernel(
         ot *= f;
 #pragma unroll
         for (int j = 0; j < kPartBatch; j++) {
-            const float wj =
-                c0 + j * kMergeParts < n_chunks ? __builtin_amdgcn_exp2f(m[j] - Mn) : 0.0f;
-            lt = fmaf(lv[j], wj, lt);
-            ot = fmaf(ov[j], wj, ot);
+            // past the last chunk: as merge_kernel
+            const bool in = c0 + j * kMergeParts < n_chunks;
+            const float wj = in ? __builtin_amdgcn_exp2f(m[j] - Mn) : 0.0f;
+            lt = fmaf(in ? lv[j] : 0.0f, wj, lt);
+            ot = fmaf(in ? ov[j] : 0.0f, wj, ot);
         }
         M = Mn;
     }

@@ -49,3 +49,36 @@ def test_empty_batch(E):  # noqa: F811
         assert np.isnan(batch_call(E, fn, gs, q, 4, 2)).all()
     for g in gs:
         g.free()
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n_kv,n_q,L,chunks", [
+    (8, 8, 100, 1), (8, 32, 100, 1), (8, 8, 640, 5), (8, 32, 640, 5), (8, 32, 1024, 8),
+    (8, 64, 1024, 8), (8, 8, 1500, 12), (4, 16, 2048, 16), (2, 8, 9000, 36)])
+def test_infinite_partials(E, d, n_kv, n_q, L, chunks):  # noqa: F811
+    """One group of V near the largest float in every token, with equal
+    scores: its sums overflow in every chunk, and both entry points return the
+    reference's infinity (a sum padded with infinity times 0 would be NaN)."""
+    rng = np.random.default_rng(0xEA4B + 820 + L)
+    data = rng.standard_normal((1, 2, n_kv, L, d), dtype=np.float32)
+    data[0, 1, 1, :, :64] = np.float32(2e38)
+    g, o = E.Cache(1, n_kv, d, L + 4), O.OracleCache(1, n_kv, d, L + 4)
+    for c in (g, o):
+        c.load_raw(data, L)
+    plan = E.fused_plan([g], n_q, n_kv)
+    say("infinite partials: plan", plan)
+    if n_cu() == 256:
+        assert plan["chunks"] == chunks
+    q = np.zeros((1, n_q, d), np.float32)
+    ref = o.attention_fused(q[0], 0, n_q, n_kv)
+    inf = np.isinf(ref)
+    assert inf.any() and np.isfinite(ref[~inf]).all()
+    outs = [batch_call(E, "eakv_attention_fused_batch_device" + s, [g], q, n_q, n_kv)[0]
+            for s in ("", "_noalloc")]
+    for out in outs:
+        assert np.array_equal(out[inf], ref[inf])
+        ok, err, bad = tol_close(out[~inf], ref[~inf])
+        assert ok, (err, bad)
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    g.free()
+    o.free()
