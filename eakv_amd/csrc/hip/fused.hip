@@ -514,20 +514,33 @@ __device__ __forceinline__ void merge_unit_p(const float *pu, const MergeOffs &m
     float res[P];
     if constexpr (!VS) {
         // softmax merge: M = max(-1e6 log2(e), m_c), l = sum l_c 2^(m_c - M),
-        // o = sum o_c 2^(m_c - M), out = o * (1/l).  Past the last chunk 0 of
-        // weight 0: the loaded o, the last chunk's, would add NaN where it is
-        // infinite.
+        // o = sum o_c 2^(m_c - M), out = o * (1/l).  The entries past the last
+        // chunk, its o of weight 0, add NaN where that is infinite: where NaN
+        // comes out, the sum is taken again with 0 there.  (0 there always
+        // costs up to 32 selects: 0.2-0.3 us a call with two outputs a thread.)
         float M = -1000000.0f * EAKV_LOG2E, lt = 0.0f, o[P];
 #pragma unroll
         for (int e = 0; e < P; e++) o[e] = 0.0f;
 #pragma unroll
         for (int j = 0; j < NB; j++) M = fmaxf(M, mv[j]);
+        float wj[NB];
 #pragma unroll
         for (int j = 0; j < NB; j++) {
-            const float wj = __builtin_amdgcn_exp2f(mv[j] - M);
-            lt = fmaf(lv[j], wj, lt);
+            wj[j] = __builtin_amdgcn_exp2f(mv[j] - M);
+            lt = fmaf(lv[j], wj[j], lt);
 #pragma unroll
-            for (int e = 0; e < P; e++) o[e] = fmaf(j < n_chunks ? ov[j][e] : 0.0f, wj, o[e]);
+            for (int e = 0; e < P; e++) o[e] = fmaf(ov[j][e], wj[j], o[e]);
+        }
+        bool nan = false;
+#pragma unroll
+        for (int e = 0; e < P; e++) nan = nan || o[e] != o[e];
+        if (nan) {
+#pragma unroll
+            for (int e = 0; e < P; e++) o[e] = 0.0f;
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int e = 0; e < P; e++) o[e] = fmaf(j < n_chunks ? ov[j][e] : 0.0f, wj[j], o[e]);
         }
 #pragma unroll
         for (int e = 0; e < P; e++) res[e] = __fadd_rn(o[e], 0.0f) * (1.0f / lt);
