@@ -1911,11 +1911,27 @@ void even_chunks(ChunkMap *cm, int n, int mc)
 // Contexts that differ little keep the even deal, whose more and smaller
 // blocks end as early (32Q/8KV, 9 of 1097-3000: 11.6 against 12.6 us; 32Q/4KV
 // d64, 32 of 1250-5000: 17.1 against 17.7): two rounds of 128-dim tokens must
-// be saved, and a quarter.
-// Returns the most chunks of a sequence, or 0 to keep the even deal, whose
-// blocks take even_rounds.
+// be saved, and a quarter.  Where the even deal is one chunk each, its blocks
+// write their results and merge nothing; the rounds saved until the last block
+// ends (`ends`; past the slots a block starts as another ends: the mean load
+// and half a chunk) then have to be worth, in units of 128 tokens of 64 dims
+// (1350 random batches of 2-32 contexts up to 24000 tokens, 15 head shapes):
+//  - the merge launch of more units than counters: 12 for one quad, 16 for two
+//    (12Q/12KV d64, 24 contexts up to 1241, 5 units saved: 12.8 against the
+//    even deal's 10.8 us; 25 up to 2743, 15 units: 14.1 against 16.8);
+//  - for two quads, whose blocks past the slots start and end with nothing
+//    beside them, 40 (d = 64: 20) for as many blocks more as there are slots
+//    (64Q/8KV d128, 31 up to 7706, 18 units for 0.9 of the slots: 52.6 against
+//    47.1; 29 of 40Q/8KV up to 5107, 45 units: 28.5 against 31.7), unless the
+//    longest context has 200 units (128Q/8KV, 16 up to 20159: 115 against 122).
+// Two-quad units that exceed the slots by themselves take a second round of
+// dispatch either way: chunks pay from 80 units in the longest context on
+// (128Q/8KV d128, 22 up to 3661: 39.4 against 34.0; 96Q/8KV, 18 up to 8279:
+// 67.4 against 78.8).
+// Returns the most chunks of a sequence, or 0 to keep the even deal of mc
+// chunks each, whose blocks take even_rounds.
 int ragged_chunks(ChunkMap *cm, const eakvd_batch *b, int vkv, int slots, int round, int hh,
-                  int gpd, int even_rounds)
+                  int gpd, int even_rounds, int mc, int64_t ctr_slots)
 {
     const int n = b->n_seq;
     int64_t sum = 0;
@@ -1943,10 +1959,31 @@ int ragged_chunks(ChunkMap *cm, const eakvd_batch *b, int vkv, int slots, int ro
         const int one_launch = (most + kInBatch - 1) / kInBatch;
         return lo < one_launch && one_launch <= lo + 2 ? one_launch : lo;
     };
+    auto blocks = [&](int r) {
+        int64_t t = 0;
+        for (int i = 0; i < n; i++) t += (rounds[i] + r - 1) / r;
+        return t * vkv;
+    };
+    // twice the rounds until blocks of r rounds have ended, times the slots
+    auto ends = [&](int r, int64_t blk) {
+        const int64_t one = 2 * (int64_t)r * slots, more = 2 * sum * vkv + (int64_t)r * slots;
+        return blk > slots && more > one ? more : one;
+    };
+    auto pays = [&](int r) {
+        if (4 * r > 3 * even_rounds || (even_rounds - r) * gpd < 4) return false;
+        if (mc > 1) return true;
+        const int64_t units = (int64_t)n * vkv, blk = blocks(r), unit = gpd * (round / 128);
+        const int64_t longest = even_rounds * unit;
+        if (hh == 2 && (units > slots || longest >= 200)) return longest >= 80;
+        const int64_t saved = (ends(even_rounds, units) - ends(r, blk)) * unit;
+        const int64_t merge = units > ctr_slots ? (hh == 1 ? 12 : 16) : 0;
+        const int64_t extra = hh == 2 && blk > slots ? blk - slots : 0;
+        return saved > 2 * (merge * slots + 20 * gpd * extra);
+    };
     int r = fit(slots / vkv);
     if (r >= 8 && 4 * (int64_t)r * slots >= 5 * sum * vkv)
         r = fit((hh == 1 ? slots + slots / 2 : 2 * slots) / vkv);
-    if (4 * r > 3 * even_rounds || (even_rounds - r) * gpd < 4) return 0;
+    if (!pays(r)) return 0;
     cm->pre[0] = 0;
     for (int i = 0; i < EAKVD_MAX_BATCH; i++)
         cm->pre[i + 1] = cm->pre[i] + (i < n ? (rounds[i] + r - 1) / r : 0);
@@ -1976,7 +2013,8 @@ FusedPlan fused_plan(const eakvd_geom *g, const eakvd_batch *b, int n_q, int n_k
         if (ragged) {
             const int round = p.wpb * p.tt;
             mc = ragged_chunks(&p.cm, b, n_kv * p.split, cu_count() * per_cu, round, p.hh,
-                               (int)g->gpd, (ml + round * p.mc - 1) / (round * p.mc));
+                               (int)g->gpd, (ml + round * p.mc - 1) / (round * p.mc), p.mc,
+                               g->ctr_slots);
         }
         p.even = mc == 0;
         if (p.even) even_chunks(&p.cm, b->n_seq, p.mc);

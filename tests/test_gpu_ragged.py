@@ -53,3 +53,29 @@ def test_ragged_batch(E, d, n_kv, n_q, lens, chunks):  # noqa: F811
     compare_sequences(os_, q[keep], out[keep], n_q, n_kv, lens)
     for g in batch:
         g.free()
+
+
+# The deals at the edges of ragged_chunks' rule where the even deal is one
+# chunk each: (d, n_kv, n_q, lens, most chunks of a sequence on 256 CUs)
+DEALS = [
+    (64, 12, 12, [1241 - 32 * i for i in range(24)], 1),     # a merge launch for 5 rounds
+    (64, 12, 12, [2743] + [700] * 24, 4),                    # and for 16
+    (128, 8, 64, [7706 - 160 * i for i in range(31)], 1),    # blocks past the slots
+    (128, 8, 64, [14435] + [2000] * 17, 8),
+    (128, 8, 128, [3661 - 120 * i for i in range(22)], 1),   # units past the slots, short
+    (128, 8, 128, [8279 - 300 * i for i in range(18)], 2),   # and long
+]
+
+
+@pytest.mark.parametrize("d,n_kv,n_q,lens,chunks", DEALS)
+def test_deal(E, d, n_kv, n_q, lens, chunks):  # noqa: F811
+    gs = []
+    for L in lens:
+        gs.append(E.Cache(1, n_kv, d, max(lens)))
+        gs[-1].advance(L)
+    plan = E.fused_plan(gs, n_q, n_kv)
+    say("deal: plan", plan)
+    if n_cu() == 256:
+        assert plan["chunks"] == chunks
+    for g in gs:
+        g.free()
