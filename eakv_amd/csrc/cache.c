@@ -172,9 +172,16 @@ int eakvi_pinned(eakv_cache_t *c, size_t n, void **p)
  * scores and output: 8Q/8KV d128 at 2048 tokens 72 us (91 with the copies), at
  * 16384 108 (129); 64Q/8KV at 77 tokens 72 (101); 32Q/8KV at 12000, where the
  * link's time for 3 MB counts, 216 (228).
+ * Inputs beyond kInPlaceMax are sent from there by the copy engine: kernels
+ * read over the link at about two thirds of its rate.  V-sum with 1.3 and 1.5 MB
+ * of weights 82 and 92 us in place, 80 and 91 sent, with 3.8 MB 177 against 156;
+ * an append of 1 MB 53 against 55, of 2 MB 110 against 96, of 4 MB 183 against
+ * 158.  Results are written in place at any size (32Q/32KV at 30000 tokens,
+ * scores of 3.8 MB, 222 against 229).
  * Larger buffers, or no pinned memory, are copied from and to pageable memory
  * by the runtime. */
 #define kPinMax ((size_t)4 << 20)
+#define kInPlaceMax ((size_t)1 << 20)
 
 void eakvi_bounce_begin(eakv_cache_t *c, size_t in_b, size_t out_b, eakvi_bounce *bo)
 {
@@ -191,6 +198,7 @@ int eakvi_bounce_in(const eakvi_bounce *bo, void *d_dst, const void *src, size_t
     if (!n) return 0;
     if (!bo->pin) return eakvd_memcpy_h2d_async(d_dst, src, n, st);
     memcpy(bo->pin, src, n);
+    if (n > kInPlaceMax) return eakvd_memcpy_h2d_async(d_dst, bo->pin, n, st);
     if (once) {
         *k_src = bo->pin;
         return 0;

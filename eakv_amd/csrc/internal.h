@@ -95,8 +95,9 @@ int  eakvi_pinned(eakv_cache_t *c, size_t n, void **p);
 /* A host-pointer call's input and result through the pinned scratch when
  * they fit (pin NULL: pageable copies to and from device memory).  begin
  * reserves in_b + out_b bytes.  in: *k_src is where the kernels read the n
- * input bytes; an input read once stays in the scratch (`once`), one that many
- * blocks read is taken to d_dst by a small kernel.  dst: where the kernels
+ * input bytes; a short input read once stays in the scratch (`once`), one that
+ * many blocks read is taken to d_dst by a small kernel, a long one by a copy.
+ * dst: where the kernels
  * write the result, given its device place.  out enqueues the copy back where
  * there is one; end copies the result out once the call's wait has succeeded
  * (rc). */

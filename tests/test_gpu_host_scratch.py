@@ -1,7 +1,7 @@
 """Host-pointer calls through the cache's pinned scratch, which the kernels read
 and write in place: every call of a series on one cache sees its own inputs and
-returns its own result, below and above the scratch's 4 MiB limit (where the
-buffers are copied instead)."""
+returns its own result, around the 1 MiB up to which an input is read there and
+around the scratch's 4 MiB limit (where the buffers are copied instead)."""
 import numpy as np
 import pytest
 
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("d,n_kv,n_q,L", [
     (128, 8, 8, 300), (64, 2, 6, 77), (128, 2, 10, 1000), (64, 32, 32, 257),
-    (128, 32, 32, 32600), (128, 32, 32, 32800)])
+    (128, 32, 32, 8190), (64, 4, 32, 8192), (128, 32, 32, 32600), (128, 32, 32, 32800)])
 def test_series_of_calls(E, d, n_kv, n_q, L):  # noqa: F811
     rng = np.random.default_rng(0xEA4B + L + d)
     rounds = 2 if L > 10000 else 6
