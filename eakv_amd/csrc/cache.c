@@ -157,9 +157,11 @@ int eakvi_pinned(eakv_cache_t *c, size_t n, void **p)
         if (c->pin) eakvd_host_free(c->pin);
         c->pin = NULL;
         c->pin_bytes = 0;
-        int e = eakvd_host_malloc(&c->pin, n);
+        /* a quarter more: scores and weights grow with every token */
+        const size_t want = n + n / 4;
+        int e = eakvd_host_malloc(&c->pin, want);
         if (e) return e;
-        c->pin_bytes = n;
+        c->pin_bytes = want;
     }
     *p = c->pin;
     return 0;

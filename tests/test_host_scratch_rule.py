@@ -84,3 +84,12 @@ def test_where_an_input_is_read(program, n, once, where):
     the result and from the caller's memory beyond."""
     place, h2d, kernels = run(program, n, once)
     assert (place, int(h2d), int(kernels)) == where
+
+
+def test_growing_needs_allocate_rarely(program):
+    """A decode loop's scores and weights grow with every token: 4096 calls that
+    each need 128 bytes more, 64 KiB to 576 KiB, allocate at most once per
+    quarter (1.25^10 > 9), and hold at most a quarter more than needed."""
+    mallocs, held, need = map(int, run(program, "grow"))
+    assert 1 <= mallocs <= 11
+    assert need <= held <= need + need // 4
