@@ -589,6 +589,10 @@ __device__ __forceinline__ void merge_unit(const float *pu, const MergeOffs &mo,
     }
 }
 
+// adjacent floats of a caller's buffer, which may be aligned to 4 bytes only
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
 // The result of a unit's only chunk: what the merge makes of one partial.
 template <bool VS>
 __device__ __forceinline__ float one_chunk(float M, float l, float o)
@@ -713,14 +717,14 @@ __device__ __forceinline__ void mfma_body(
     for (int hq = 0; hq < HH; hq++) {
         qrow[hq] = 4 * hq + ha < G;
         if (w != hq) continue;
-        const float4 *qh4 = (const float4 *)(qs + (qrow[hq] ? 4 * hq + ha : 0) * D);
+        const f4u *qh4 = (const f4u *)(qs + (qrow[hq] ? 4 * hq + ha : 0) * D);
 #pragma unroll
         for (int gg = 0; gg < GPD; gg++)
 #pragma unroll
             for (int h2 = 0; h2 < 2; h2++)
 #pragma unroll
                 for (int v4 = 0; v4 < 2; v4++) {
-                    const float4 f = qh4[(64 * gg + 32 * h2 + 8 * qq) / 4 + v4];
+                    const f4u f = qh4[(64 * gg + 32 * h2 + 8 * qq) / 4 + v4];
                     float *d = &qv[hq][gg][8 * h2 + 4 * v4];
                     d[0] = f.x; d[1] = f.y; d[2] = f.z; d[3] = f.w;
                 }
@@ -1329,8 +1333,8 @@ __device__ __forceinline__ void mfma_body(
             o1 = fmaf(ov.y, f, o1);
         }
         if (n_chunks == 1) {
-            *reinterpret_cast<float2 *>(ou + h * D + dim) =
-                make_float2(one_chunk<VS>(M, lt, o0), one_chunk<VS>(M, lt, o1));
+            *reinterpret_cast<f2u *>(ou + h * D + dim) =
+                f2u{one_chunk<VS>(M, lt, o0), one_chunk<VS>(M, lt, o1)};
             continue;
         }
         float *dst = pu + (h * nb + ch) * (D + 2);

@@ -82,3 +82,47 @@ def test_infinite_partials(E, d, n_kv, n_q, L, chunks):  # noqa: F811
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
     g.free()
     o.free()
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n_q,L", [(8, 100), (32, 100), (64, 100), (32, 1024), (64, 1500),
+                                   (32, 4096)])
+def test_buffers_aligned_to_4_bytes(E, d, n_q, L):  # noqa: F811
+    """Queries, weights, outputs and scores at addresses that are only 4-byte
+    aligned, one chunk (stored from the chunk itself) and several: the same bits
+    as at aligned addresses, and nothing beside the results touched."""
+    from eakv_amd.hipmem import DeviceArray
+    n_kv = 8
+    rng = np.random.default_rng(0xEA4B + 830 + L + n_q)
+    g = E.Cache(1, n_kv, d, L + 4)
+    g.load_raw(rng.standard_normal((1, 2, n_kv, L, d), dtype=np.float32), L)
+    q = rng.standard_normal((n_q, d), dtype=np.float32)
+    w = rng.random((n_q, L), dtype=np.float32)
+    one = np.zeros(1, np.float32)
+    dq = DeviceArray.from_host(np.concatenate([one, q.ravel()]))
+    dq0 = DeviceArray.from_host(q)
+    dw = DeviceArray.from_host(np.concatenate([one, w.ravel()]))
+    dw0 = DeviceArray.from_host(w)
+    lib, hs = E.lib(), E.handles([g])
+    q_at, w_at = (dq0.ptr, dq.ptr + 4), (dw0.ptr, dw.ptr + 4)
+    calls = [
+        (n_q * d, lambda i, p: lib.eakv_attention_fused_batch_device(
+            hs, 1, 0, q_at[i], n_q, n_kv, p, None)),
+        (n_q * d, lambda i, p: lib.eakv_attention_fused_batch_device_noalloc(
+            hs, 1, 0, q_at[i], n_q, n_kv, p, None)),
+        (n_q * d, lambda i, p: lib.eakv_attention_output_device(
+            g.h, w_at[i], 0, n_q, n_kv, p, None)),
+        (n_q * L, lambda i, p: lib.eakv_attention_scores_device(
+            g.h, q_at[i], 0, n_q, n_kv, p, None)),
+    ]
+    for n, call in calls:
+        outs = []
+        for off in (0, 1):
+            buf = DeviceArray.from_host(np.full(n + 2, 7.0, np.float32))
+            assert call(off, buf.ptr + 4 * off) == 0, E.last_error()
+            g.sync()
+            got = buf.download()
+            assert got[n + off] == 7.0 and (off == 0 or got[0] == 7.0)
+            outs.append(got[off:n + off].view(np.uint32))
+        assert np.array_equal(*outs)
+    g.free()
