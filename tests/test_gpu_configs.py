@@ -47,24 +47,14 @@ def pair(E, nl, nh, hd, lmax):
     return E.Cache(nl, nh, hd, lmax), O.OracleCache(nl, nh, hd, lmax)
 
 
-def n_cu():
-    lib = C.CDLL(os.path.join(ROOT, "eakv_amd", "libeakv_synth.so"))
-    lib.eakv_synth_cu_count.restype = C.c_int
-    return lib.eakv_synth_cu_count() or 256
-
-
-def mfma_chunks(L, units, qpk, d):
-    """Chunks per (sequence, kv head) of the fused matrix-core program: the
-    launch rule of fused.hip's mfma_blocks_per_unit (chunks of at least 512
-    tokens, 256 when that leaves fewer blocks than CUs; resident blocks per
-    CU: 2 for up to 4 q heads per kv head, else 1 at d=128, 2 at d=64)."""
-    per_cu = 2 if qpk <= 4 else (1 if d == 128 else 2)
-    cu = n_cu()
-    slots = cu * per_cu
-    nb = 1 if units >= slots else slots // units
-    coarse = -(-L // 512)
-    cap = -(-L // 256) if units * coarse < cu else coarse
-    return max(1, min(nb, cap))
+def launch_plan(E, L, n_q, n_kv, d):
+    """The fused call's launch for one cache of L tokens, as the library plans it."""
+    c = E.Cache(1, n_kv, d, L)
+    c.advance(L)
+    plan = E.fused_plan([c], n_q, n_kv)
+    c.free()
+    assert plan["mfma"] == 1
+    return plan
 
 
 def unfused_check(g, o, q, layer, n_q, n_kv, rng, signed=True):
@@ -300,17 +290,6 @@ def test_blocks_beyond_1gib(E, rng, nkv, n_q, d, lmax, L):
     g.free()
 
 
-# -------------------------------------------- long contexts: 8-part merge
-
-def tile_tokens(L, units, qpk, d):
-    """Tokens per tile of the fused matrix-core program (fused.hip's
-    tile_tokens): 64 where waves serve two quads (5-8 q heads per kv head)
-    and each of the unit's 8 waves per chunk gets at least 4 tiles of 64,
-    else 32."""
-    mc = mfma_chunks(L, units, qpk, d)
-    return 64 if qpk > 4 and -(-L // 64) >= 4 * mc * 8 else 32
-
-
 # ------------------------------------------ 64-token tiles (two-quad waves)
 
 @pytest.mark.parametrize("d,n_q,n_kv,L,case", [
@@ -323,7 +302,7 @@ def test_64_token_tiles(E, rng, d, n_q, n_kv, L, case):
     scores that rise along the context (the running max moves), and the
     V-sum mode with signed weights (the V-sum's grid has the same chunks,
     so it runs 64-token tiles too)."""
-    assert tile_tokens(L, n_kv, n_q // n_kv, d) == 64
+    assert launch_plan(E, L, n_q, n_kv, d)["tile_tokens"] == 64
     say("tt64", d, n_q, n_kv, L, case)
     if case == "slope":
         u = rng.standard_normal((n_kv, d))
@@ -361,7 +340,7 @@ def test_long_context_nonfinite_values(E, rng, d, n_q, n_kv, L, where):
     """A NaN first value of a group in K (every output of the kv head's q heads
     NaN) or V (that group's 64 dims NaN) with more than 16 chunks per
     sequence, so the chunk merge is the 8-part one."""
-    assert mfma_chunks(L, n_kv, n_q // n_kv, d) > 16
+    assert launch_plan(E, L, n_q, n_kv, d)["chunks"] > 16
     say("long-nan", d, n_q, n_kv, L, where)
     data = rng.standard_normal((1, 2, n_kv, L, d)).astype(np.float32)
     data[0, 0 if where == "k" else 1, 1, (2 * L) // 3, 0] = np.nan
@@ -384,7 +363,7 @@ def test_long_context_moving_max(E, rng, d, n_q, n_kv, L, slope):
     """Scores rising (the running max moves in chunk after chunk) or falling
     over a context of more than 16 chunks: the 8-part merge rescales every
     part to the common max."""
-    assert mfma_chunks(L, n_kv, n_q // n_kv, d) > 16
+    assert launch_plan(E, L, n_q, n_kv, d)["chunks"] > 16
     say("long-slope", d, n_q, n_kv, L, slope)
     u = rng.standard_normal((n_kv, d))
     u /= np.linalg.norm(u, axis=1, keepdims=True)

@@ -1,8 +1,9 @@
 """The K-score of groups of q heads (k_score_mfma_kernel, hip/kscore.hip), whose
 dots run on the matrix cores, bit for bit against the oracle: group sizes around
 its quads of heads, contexts around its 256-token slices and long enough for
-two quads a wave (every slice of every quad more than three blocks per CU), and
-values with denormal products."""
+two quads a wave (every slice of every quad more than three blocks per CU; at
+20000 tokens a block takes several slices, with 10 heads a group the last block's
+second quad is empty), and values with denormal products."""
 import numpy as np
 import pytest
 
@@ -16,7 +17,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n_kv,qpk,L,tiny", [
     (2, 2, 1, False), (1, 3, 255, False), (3, 4, 256, False), (2, 5, 257, False),
     (1, 8, 1000, True), (2, 9, 513, False), (1, 17, 300, False),
-    (8, 8, 49 * 256 + 1, False), (16, 6, 25 * 256 - 1, False), (8, 4, 27000, False)])
+    (8, 8, 49 * 256 + 1, False), (16, 6, 25 * 256 - 1, False), (8, 4, 27000, False),
+    (8, 8, 20000, False), (4, 10, 20000, False)])
 def test_group_scores_bit_exact(E, d, n_kv, qpk, L, tiny):  # noqa: F811
     rng = np.random.default_rng(0xEA4B + 31 * qpk + L + d)
     data = np.stack([chan_k(rng, n_kv, L, d), rng.standard_normal((n_kv, L, d), dtype=np.float32)])

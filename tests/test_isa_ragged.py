@@ -37,7 +37,11 @@ def test_groups_and_waits(kernels, d, hh, tt):
     gpd = d // 64
     n_scale, n_v, n_reg = max(4 * tt * gpd * 4, 1024) // 1024, tt * 32 * gpd // 1024, tt // 16 * gpd
     body = kernels[(d, hh, tt)]
-    loop = [(lb, tk) for lb, tk in isa.blocks(body) if tk][1:]
+    with_loads = [(lb, tk) for lb, tk in isa.blocks(body) if tk]
+    # prologue: the 4-byte prime load of a V slot and the first scale load
+    # come first (the first explicit wait needs exactly those two)
+    assert with_loads[0][1].startswith("DD"), with_loads[0]
+    loop = with_loads[1:]
     assert loop
     group = "D" * (n_v + n_scale) + "g" * n_reg
     for lb, tk in loop:
@@ -46,7 +50,7 @@ def test_groups_and_waits(kernels, d, hh, tt):
     assert isa.check_waits(loop, n_v, n_scale, n_reg) >= 1
 
 
-def test_no_scratch():
+def test_no_scratch(kernels):
     metas = open(isa.ASM).read().split("  - .agpr_count:")[1:]
     seen = 0
     for m in metas:
