@@ -145,7 +145,7 @@ int eakvd_fused(const eakvd_geom *g, const eakvd_batch *b, int layer,
 /* The launch eakvd_fused makes for this batch, head split and counter
  * region (ctr as eakvd_fused's): out[0] 1 for the matrix-core program (0:
  * the VALU program), [1] the most chunks of a (sequence, virtual kv head) unit, [2] 1
- * when the chunks merge inside the launch (0: a merge launch follows), [3]
+ * when the chunks merge inside the launch (0: in a merge launch, where [1] > 1), [3]
  * tokens per tile, [4] waves per block, [5] the most tiles a wave walks,
  * [6] quads of q heads per wave, [7] virtual kv heads per kv head. */
 void eakvd_fused_plan(const eakvd_geom *g, const eakvd_batch *b, int n_q, int n_kv,

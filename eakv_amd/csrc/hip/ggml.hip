@@ -295,10 +295,13 @@ extern "C" int eakvd_ggml_vec_dot(int n, float *s, size_t bs, const void *vx, si
 {
     if (nrc <= 0) return 0;
     // One vector for all rows, whole in LDS (up to 64 KB): from 2048 rows on,
-    // where the copy of y into LDS is made up for (100 rows of 11008: 18.3
-    // against 18.5 us), with as few lanes a row as still fill the chip's SIMDs
-    // about twice (8192 rows of 4096: 9.7 us with 16 lanes, 10.4 with 8, 13.4
-    // with 4; 32768 of 1024: 10.1, 7.7, 6.7).
+    // where it is never slower by more than 1 % (2048 rows of 16384 26.2 against
+    // 26.1 us, of 4096 8.6 against 8.8; 3072 of 16384 27.8 against 36.9).  Below,
+    // the copy of y into LDS is not always made up for (64 rows of 16384 25.4
+    // against 24.0, 1024 26.2 against 25.7, though 512 26.0 against 28.2).  With
+    // as few lanes a row as still fill the chip's SIMDs about twice (8192 rows of
+    // 4096: 9.7 us with 16 lanes, 10.4 with 8, 13.4 with 4; 32768 of 1024: 10.1,
+    // 7.7, 6.7).
     if (by == 0 && nrc >= 2048 && n >= 64 && n <= 16384) {
         const int lpr = nrc >= 32768 ? 4 : nrc >= 16384 ? 8 : 16;
         auto kern = lpr == 4 ? ggml_mat_vec_kernel<4> : lpr == 8 ? ggml_mat_vec_kernel<8>

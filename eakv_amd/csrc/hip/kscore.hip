@@ -17,10 +17,10 @@
 // several 256-token slices with the next slice's loads in flight while it
 // computes the current one.  Nibbles become floats by masking a dword to four
 // byte-wide nibbles and converting its bytes (v_cvt_f32_ubyte0..3): exact,
-// as the reference's int-to-float conversion of the nibble.  Grids that
-// leave the chip unfilled split the work further: a group's q heads over
-// blocks, or (one q head per kv head) a token's 16 accumulators over four
-// lanes (k_score_mha4_kernel).
+// as the reference's int-to-float conversion of the nibble.  Short contexts
+// split the work further: a group's quads of q heads over blocks, or (one q
+// head per kv head) a token's 16 accumulators over four lanes
+// (k_score_mha4_kernel).
 #include "common.h"
 
 namespace {
@@ -281,11 +281,10 @@ __global__ __launch_bounds__(256) void k_score_mha4_kernel(
 // i's dim of chunk c, and 8 registers hold four heads' q.  A lane ends with the
 // 16 accumulators of its own token and four heads, summed by the reference's
 // tree without leaving the lane.
-// What bounds it: issue.  Per 64 tokens and four heads 128 MFMAs of 8.9 cycles
+// What bounds it: issue.  Per 64 tokens and four heads 128 MFMAs of 8.1 cycles
 // and 128 dequantizations of about 8 (a conversion takes 4.4 cycles, an FMA of
-// vector operands 2.8); with the q values as scalar operands of vector FMAs
-// (4.3 cycles each) the same took 3,400 cycles instead of 2,400, and waited
-// for scalar loads.  Per K-score and V-sum call of a layer: 32Q/8KV d128 at
+// vector operands 2.6): 2,100 cycles; with the q values as scalar operands of
+// vector FMAs (4.3 cycles each) 3,200, and it waited for scalar loads.  Per K-score and V-sum call of a layer: 32Q/8KV d128 at
 // 30011 tokens 17.3 against 21.2 us, 64Q/8KV at 100000 53.8 against 73.9,
 // 16Q/8KV at 20000 14.3 against 16.4, 32Q/4KV d64 at 60000 15.9 against 19.3;
 // launch-bound sizes (up to 5000 tokens) are the same.
@@ -327,9 +326,9 @@ __device__ __forceinline__ void k_macs(KAcc<NQ> &acc, const float (*A)[D / 16], 
 }
 
 // The fences keep a chunk's MFMAs in one run: matrix and vector instructions of
-// a SIMD do not overlap, and each change between them costs about 5 cycles (a
-// 4x4x1 takes 8.9 cycles; one with two vector FMAs 14.0 in runs of 16, 18.9
-// taken in turn).
+// a SIMD do not overlap, and each change between them costs cycles (a 4x4x1
+// takes 8.1; one with two vector FMAs of 2.6 takes 12.8 to 13.9 in runs of 16,
+// 16.1 to 18.9 taken in turn).
 template <int C, int D, int NQ>
 __device__ __forceinline__ void k_chunks(KAcc<NQ> &acc, const float (*A)[D / 16],
                                          const KTok<D> &T)

@@ -120,8 +120,9 @@ int eakv_attention_fused_batch_device(eakv_cache_t *const *caches,
  * partials in the library's static device scratch of 16 MiB per device
  * instead of caches[0]'s workspace, so no call path allocates.  Same
  * arguments, results and stream ordering; EAKV_ERR_INVALID when the launch
- * would need more than 16 MiB of partials (n_caches * n_q_heads * chunks *
- * (head_dim + 2) * 4 bytes: 1.1 MB for 8 caches of 32 q heads over 32K
+ * would need more than 16 MiB of partials (n_q_heads * (head_dim + 2) * 4
+ * bytes for every chunk of every cache; each cache has the same number of
+ * chunks, or, where context lengths differ, a number in proportion: 1.1 MB for 8 caches of 32 q heads over 32K
  * tokens, 1.1 MB for 64 q heads over 128K tokens).
  * Every call on one device shares that scratch: calls that overlap in time
  * on one device race, and ordering them is the caller's. */
@@ -137,10 +138,10 @@ int eakv_attention_fused_batch_device_noalloc(eakv_cache_t *const *caches,
  * current seq_len and this head split, for diagnostics and tests; nothing is
  * launched.  plan (8 entries): [0] 1 for the matrix-core program, 0 for the
  * VALU program (layer blocks beyond 32-bit buffer offsets); [1] the most
- * chunks of a (sequence, kv head) unit; [2] 1 when the chunks are merged inside the
- * launch (up to 16 chunks per unit), 0 when a merge launch follows; [3]
- * tokens per tile; [4] waves per
- * block; [5] the most tiles one wave walks; [6] quads of q heads per wave;
+ * chunks of a (sequence, kv head) unit; [2] 1 when a unit's chunks are merged
+ * inside the launch (up to 16 chunks per unit, and a counter for every unit),
+ * else 0: a merge launch follows where [1] is above 1; [3] tokens per tile; [4]
+ * waves per block; [5] the most tiles one wave walks; [6] quads of q heads per wave;
  * [7] virtual kv heads per kv head (groups above 8 q heads). */
 int eakv_attention_fused_plan(eakv_cache_t *const *caches, int n_caches, int n_q_heads,
                               int n_kv_heads, int noalloc, int32_t *plan);
